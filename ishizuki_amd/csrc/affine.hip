@@ -612,11 +612,13 @@ extern "C" int ishz_affine_matmul(const void *x, int x_dtype, int M, int K, cons
   hipStream_t st = S(stream);
   if (x_dtype == ISHZ_DT_F32 || (group != 64 && group != 128))
     return affine_precise(x, x_dtype, M, K, codes, scales, biases, scale_dtype == ISHZ_DT_BF16, N, bits, group, y, st);
-  StreamTemp tmp(st);  // bf16 activations: their fp16 image
-  if (x_dtype != ISHZ_DT_F16 && (rc = tmp.get(act_image_bytes(M, K)))) return rc;
-  const uint16_t *xh;
-  const float *rs;
-  if ((rc = act_prepare(x, x_dtype, M, K, tmp.p, st, &xh, &rs))) return rc;
+  StreamTemp tmp(st);  // bf16 rows: their fp16 image (one row: the GEMV makes it while staging x)
+  const uint16_t *xh = (const uint16_t *)x;
+  const float *rs = nullptr;
+  if (M > 1) {
+    if (x_dtype != ISHZ_DT_F16 && (rc = tmp.get(act_image_bytes(M, K)))) return rc;
+    if ((rc = act_prepare(x, x_dtype, M, K, tmp.p, st, &xh, &rs))) return rc;
+  }
   const Out o{y, x_dtype, rs};
   if (bits != 2)
     return affine_nbit_dispatch(xh, M, K, codes, scales, biases, scale_dtype == ISHZ_DT_BF16, N, bits, group, o, st);
@@ -657,9 +659,9 @@ extern "C" int ishz_affine_linear(const void *x, int x_dtype, int M, int K, cons
     }
     if (x_dtype == ISHZ_DT_F32 || (group != 64 && group != 128))
       return affine_precise(xr, x_dtype, M, K, codes, scales, biases, bf16s, N, bits, group, y, st);
-    const uint16_t *xh;
-    const float *rs;
-    if ((rc = act_prepare(xr, x_dtype, M, K, img, st, &xh, &rs))) return rc;
+    const uint16_t *xh = (const uint16_t *)xr;
+    const float *rs = nullptr;
+    if (M > 1 && (rc = act_prepare(xr, x_dtype, M, K, img, st, &xh, &rs))) return rc;  // (M = 1: by the GEMV)
     const Out o{y, x_dtype, rs};
     if (bits != 2) return affine_nbit_dispatch(xh, M, K, codes, scales, biases, bf16s, N, bits, group, o, st);
     return affine_dispatch(xh, M, K, nullptr, 0, codes, scales, biases, bf16s, N, group, o, st);

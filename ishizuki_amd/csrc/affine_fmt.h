@@ -227,7 +227,8 @@ struct FAffine {
   }
   // Rotates and stages passes c0, c0 + nw, ... (PF of them) of this wave from their loads, into
   // LDS or (prestage) into the global image.
-  static DEV void stage_group(const Args &a, u4 *xs, float *xsum, int c0, int nw, const XPre &cur) {
+  // down: bf16 x (never rotated here) is staged as fp16(x * down); 0: x is fp16.
+  static DEV void stage_group(const Args &a, u4 *xs, float *xsum, int c0, int nw, const XPre &cur, float down = 0.0f) {
     const int lane = threadIdx.x & 63;
     const int bl = a.block;
     const float scale = bl > 1 ? 1.0f / __builtin_sqrtf((float)bl) : 1.0f;
@@ -237,9 +238,10 @@ struct FAffine {
       if (c0 + j * nw >= npass) break;
       const int k = (c0 + j * nw) * 512 + 8 * lane;
       float v[8];
+      const u4 xv = down != 0.0f ? bf16_to_half8(cur.xv[j], down) : cur.xv[j];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const h2 hv = as_h2(cur.xv[j][e]);
+        const h2 hv = as_h2(xv[e]);
         v[2 * e] = (float)hv.x;
         v[2 * e + 1] = (float)hv.y;
       }
@@ -253,7 +255,18 @@ struct FAffine {
     if (a.block > 128) return p;
     return load_group(a, x, threadIdx.x >> 6, blockDim.x >> 6);
   }
-  static DEV void stage(const Args &a, const uint16_t *x, u4 *xs, float *xsum, u4 *extra, int, const XPre &pre) {
+  // The exponent of a bf16 row's largest magnitude (GgmlGemv::bf16_scale).
+  static DEV int bf16_scale(const uint16_t *x, int units, const XPre &pre, uint32_t *scratch) {
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6, npass = (units * 64 + 511) / 512;
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < PF; j++) m = bf16_absmax(pre.xv[j], m);
+    for (int c = wave_id() + PF * nw; c < npass; c += nw)
+      m = bf16_absmax(*(const u4 *)(x + min(c * 512 + 8 * lane, units * 64 - 8)), m);
+    return bf16_row_exponent(block_absmax(m, scratch));
+  }
+  static DEV void stage(const Args &a, const uint16_t *x, u4 *xs, float *xsum, u4 *extra, int, const XPre &pre,
+                        float down = 0.0f) {
     const int lane = threadIdx.x & 63, wave = wave_id(), nw = blockDim.x >> 6;
     if (a.block > 128) {
       uint16_t *xh = (uint16_t *)xs;
@@ -270,9 +283,9 @@ struct FAffine {
       return;
     }
     const int npass = (a.K + 511) / 512;
-    stage_group(a, xs, xsum, wave, nw, pre);  // first group: loads issued by stage_load
+    stage_group(a, xs, xsum, wave, nw, pre, down);  // first group: loads issued by stage_load
     for (int c0 = wave + PF * nw; c0 < npass; c0 += PF * nw)
-      stage_group(a, xs, xsum, c0, nw, load_group(a, x, c0, nw));
+      stage_group(a, xs, xsum, c0, nw, load_group(a, x, c0, nw), down);
     __syncthreads();
   }
 

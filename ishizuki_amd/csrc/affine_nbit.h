@@ -150,9 +150,6 @@ struct FAffineN : GgmlGemv<FAffineN<BITS, GS, BF16S>> {
     Base::load_sums(x, units, threadIdx.x, p.sv);
     return p;
   }
-  static DEV void stage(const Args &, const uint16_t *x, u4 *xs, float *xsum, u4 *extra, int units, const XPre &pre) {
-    Base::stage_body(x, xs, xsum, extra, units, pre);
-  }
 
   // Streaming MFMA verify: quarter g of step j is unit 4j + g of the chunk; one scale group per
   // quarter (VNS = 1, eight MFMAs).

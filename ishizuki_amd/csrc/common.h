@@ -130,6 +130,60 @@ DEV float group_sum(float v) {
   return v;
 }
 
+// ---------------------------------------------------------------- bf16 rows as fp16 images
+// The larger of m and the magnitudes of eight bf16 values, as bf16 bits (an unsigned compare of the
+// bits without their sign; a NaN is larger than infinity).
+DEV uint32_t bf16_absmax(u4 v, uint32_t m) {
+  typedef uint16_t us2 __attribute__((ext_vector_type(2)));
+  us2 a = __builtin_bit_cast(us2, v.x & 0x7fff7fffu);
+#pragma unroll
+  for (int i = 1; i < 4; i++) a = __builtin_elementwise_max(a, __builtin_bit_cast(us2, v[i] & 0x7fff7fffu));
+  return max(m, max((uint32_t)a.x, (uint32_t)a.y));
+}
+// The maximum over the wave's lanes.
+DEV uint32_t wave_absmax(uint32_t m) {
+#define ISHZ_DPPU(ctrl) m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, ctrl, 0xf, 0xf, true))
+  ISHZ_DPPU(0xB1);
+  ISHZ_DPPU(0x4E);
+  ISHZ_DPPU(0x141);
+  ISHZ_DPPU(0x140);
+#undef ISHZ_DPPU
+  const auto a = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+  m = max((uint32_t)a[0], (uint32_t)a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+  return max((uint32_t)b[0], (uint32_t)b[1]);
+}
+// The maximum over the workgroup's threads; scratch: one LDS word per wave, free again on return.
+DEV uint32_t block_absmax(uint32_t m, uint32_t *scratch) {
+  m = wave_absmax(m);
+  if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = 0;
+  for (int w = 0; w < (int)(blockDim.x >> 6); w++) m = max(m, scratch[w]);
+  __syncthreads();
+  return m;
+}
+// e of 2^(e-1) <= m < 2^e for a row whose largest magnitude has bf16 bits m; 0 for a row of zeros or
+// with an infinity or a NaN. At most 127, so that 2^e stays a finite fp32 factor (a row whose
+// largest value lies in (2^127, FLT_MAX] lands in [0.5, 2)).
+DEV int bf16_row_exponent(uint32_t m) {
+  if (m == 0 || m >= 0x7f80u) return 0;
+  int e;
+  (void)frexpf(__builtin_bit_cast(float, m << 16), &e);
+  return min(e, 127);
+}
+// Eight bf16 values times `down`, rounded to fp16.
+DEV u4 bf16_to_half8(u4 v, float down) {
+  u4 o;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float lo = __builtin_bit_cast(float, v[i] << 16), hi = __builtin_bit_cast(float, v[i] & 0xffff0000u);
+    o[i] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(lo * down)) |
+           (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(hi * down)) << 16;
+  }
+  return o;
+}
+
 // Value of lane K of each quad (DPP quad_perm [K,K,K,K]).
 template <int K>
 DEV uint32_t quad_bcast(uint32_t v) {
@@ -189,13 +243,13 @@ int decline(const std::string &why);
 int einval(const std::string &why);
 inline hipStream_t S(ishz_stream_t s) { return (hipStream_t)s; }
 
-// Activations other than fp16 (bf16, fp32) are converted once per call into an fp16 image with a
-// power-of-two factor per row, and every kernel stages that image as it stages fp16 x:
+// bf16 activations are converted once per call into an fp16 image with a power-of-two factor per
+// row, and every kernel stages that image as it stages fp16 x:
 //   xh[m][k] = fp16(x[m][k] * 2^-e_m),  2^(e_m - 1) <= max_k |x[m][k]| < 2^e_m,
 // outputs multiplied back by rs[m] = 2^e_m (exact) in fp32 before their one narrowing to x's
 // dtype. bf16 values (8 significant bits) land exactly down to 2^-17 of their row's largest
-// (fp16 subnormals below 2^-14 still hold 8 bits there); smaller ones within 2^-25 of it. fp32
-// values round to fp16 (2^-11 relative). The image: act_image_bytes(M, K) bytes of a workspace.
+// (fp16 subnormals below 2^-14 still hold 8 bits there); smaller ones within 2^-25 of it. The
+// image: act_image_bytes(M, K) bytes of a workspace.
 size_t act_image_bytes(int M, int K);
 int act_prepare(const void *x, int dt, int M, int K, void *image, hipStream_t st, const uint16_t **xh,
                 const float **rs);

@@ -97,6 +97,13 @@ template <class F>
 __host__ __device__ constexpr bool gemv_interleaved() {
   return !gemv_has_prepare<F>() && !gemv_has_store<F>() && !gemv_multi_x<F>() && !gemv_has_align<F>();
 }
+// bf16 x (formats without those hooks whose staging takes it): the workgroup turns the raw row it
+// stages into the fp16 image itself, with the row's power-of-two factor (F::bf16_scale), instead of
+// reading an image another launch wrote.
+template <class F>
+__host__ __device__ constexpr bool gemv_bf16_x() {
+  return gemv_interleaved<F>() && requires { &F::bf16_scale; };
+}
 template <class F>
 __host__ __device__ int gemv_align(const typename F::Args &a, int rpw) {
   if constexpr (gemv_has_align<F>()) return F::group_align(a, rpw);
@@ -115,7 +122,7 @@ __host__ __device__ constexpr int gemv_threads() {
   else return 256;
 }
 
-template <class F, int LPR, int D, bool RAGGED, bool BIG = false>
+template <class F, int LPR, int D, bool RAGGED, bool BIG = false, bool XBF = false>
 __global__ __launch_bounds__((gemv_threads<F, LPR, BIG>())) void gemv_kernel(typename F::Args args, const uint16_t *__restrict__ x,
                                                    Out out, int nwg, int part_off) {
   static_assert(LPR % 16 == 0, "lanes per row must be a multiple of 16");
@@ -180,7 +187,7 @@ __global__ __launch_bounds__((gemv_threads<F, LPR, BIG>())) void gemv_kernel(typ
   uint64_t ts[5];
   ts[0] = __builtin_amdgcn_s_memrealtime();
 #endif
-  const typename F::XPre pre = F::stage_load(args, x, units);
+  typename F::XPre pre = F::stage_load(args, x, units);
   typename F::Raw buf[D];
   int gl = gf + (T ? tb / upl : 0), kl = T ? tb % upl : 0;
   const int gc0 = gl, kc0 = kl;
@@ -190,6 +197,14 @@ __global__ __launch_bounds__((gemv_threads<F, LPR, BIG>())) void gemv_kernel(typ
     advance(gl, kl);
   }
 
+  // XBF (its own instantiation: a branch here cost the fp16 2-bit GEMV 0.5 %): raw bf16 x, staged as
+  // fp16(x * down), outputs times `up`
+  float down = 0.0f, up = 1.0f;
+  if constexpr (XBF) {
+    const int e = F::bf16_scale(x, units, pre, (uint32_t *)smem);
+    down = ldexpf(1.0f, -e);
+    up = ldexpf(1.0f, e);
+  }
   // after the first loads are out (visible after staging's barrier)
   for (int i = threadIdx.x; i < WPG * nrows; i += WPG * 64) part[i] = 0.0f;
   int im0 = 0;  // first x image of this workgroup's rows
@@ -198,6 +213,8 @@ __global__ __launch_bounds__((gemv_threads<F, LPR, BIG>())) void gemv_kernel(typ
   } else if constexpr (gemv_multi_x<F>()) {
     im0 = F::xsel(args, min(gf * RPW, N - 1));
     F::stage(args, x, xs, xsum, extra, units, pre, im0, F::xsel(args, min(max(gend * RPW - 1, gf * RPW), N - 1)));
+  } else if constexpr (XBF) {
+    F::stage(args, x, xs, xsum, extra, units, pre, down);  // ends with a barrier
   } else {
     F::stage(args, x, xs, xsum, extra, units, pre);  // ends with a barrier
   }
@@ -264,7 +281,10 @@ __global__ __launch_bounds__((gemv_threads<F, LPR, BIG>())) void gemv_kernel(typ
     if constexpr (gemv_has_store<F>()) part[i] = s;  // only this thread reads row i's partials
     else if (IL) {
       const int r = phys(i / RPW) * RPW + i % RPW;
-      if (r < N) out.put(r, 0, s);
+      if (r < N) {
+        if constexpr (XBF) store_act(out.y, r, ISHZ_DT_BF16, s * up);
+        else out.put(r, 0, s);
+      }
     } else if (gf * RPW + i < N) out.put(gf * RPW + i, 0, s);
   }
   if constexpr (gemv_has_store<F>()) {
@@ -281,8 +301,10 @@ int gemv_num_cu();
 // Grid: one resident round of workgroups (at most what the compiled kernel's registers and this
 // launch's LDS allow), each an equal share of row groups. LDS: the staged x images and sums, the
 // format's tables, then the waves' partial dots for the workgroup's rows.
-template <class F, int LPR, bool RAGGED, bool BIG = false>
+template <class F, int LPR, bool RAGGED, bool BIG = false, bool XBF = false>
 static int launch_gemv_k(const typename F::Args &a, const void *x, const Out &o, hipStream_t st) {
+  if constexpr (gemv_bf16_x<F>() && !XBF)
+    if (o.dt == ISHZ_DT_BF16 && !o.rs) return launch_gemv_k<F, LPR, RAGGED, BIG, true>(a, x, o, st);
   constexpr int RPW = 64 / LPR;
   constexpr int NT = gemv_threads<F, LPR, BIG>(), WPG = NT / 64;
   const int units = F::units(a.K);
@@ -290,7 +312,7 @@ static int launch_gemv_k(const typename F::Args &a, const void *x, const Out &o,
   const size_t xlds = gemv_nx<F>(a) * (ug * 16 * F::R * 16 + ug * 16 * F::Q * 4) + F::extra_lds_bytes(a);
   const size_t part_off = (xlds + 15) / 16 * 16;
   if (part_off > 160 * 1024) return decline("K too large for the GEMV's LDS copy of x");
-  auto kern = gemv_kernel<F, LPR, F::RING, RAGGED, BIG>;
+  auto kern = gemv_kernel<F, LPR, F::RING, RAGGED, BIG, XBF>;
   const int GA = gemv_align<F>(a, RPW), groups = (a.N + RPW - 1) / RPW, units_g = (groups + GA - 1) / GA;
   const int wg_cap = std::max(F::occ(a) * 4 / WPG, 1);  // workgroups per CU the grid is sized for
   int nwg = 0;
@@ -321,7 +343,7 @@ static int launch_gemv_k(const typename F::Args &a, const void *x, const Out &o,
 // 1024-thread workgroups (at K = 25600, N = 5120 on MI355X: Q4_K 20.7 -> 19.8 us, Q6_K 28.0 ->
 // 27.5, IQ2_XS 20.4 -> 18.8 against 64 lanes per row, whose last slot was 12 % padding). RAGGED:
 // the row's units are not a whole number of every lane's slots. x is fp16 (or an activation image, with its row
-// factor in rs); y in dtype odt.
+// factor in rs), or raw bf16 where odt is bf16 and rs null (gemv_bf16_x formats); y in dtype odt.
 template <class F>
 static int launch_gemv(const typename F::Args &a, const void *x, void *y, hipStream_t st, int odt = ISHZ_DT_F16,
                        const float *rs = nullptr) {

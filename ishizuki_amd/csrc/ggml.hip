@@ -331,7 +331,8 @@ static int verify(const void *x, int M, int K, const void *w, int N, const Out &
 
 template <class F>
 static int gemv(const void *x, int K, const void *w, int N, const Out &y, hipStream_t st) {
-  if (K % F::GEMV_K_MULT) return verify<F>(x, 1, K, w, N, y, st);
+  if constexpr (F::GEMV_K_MULT != F::BS)
+    if (K % F::GEMV_K_MULT) return verify<F>(x, 1, K, w, N, y, st);
   const typename F::Args a{(const uint8_t *)w, (size_t)(K / F::BS) * F::TS, K, N};
   return launch_gemv<F>(a, x, y.y, st, y.dt, y.rs);
 }
@@ -417,6 +418,17 @@ static int ggml_call(uint32_t type, const void *x, int x_dtype, int M, int K, co
 #undef X
     }
     return decline("unsupported GGML type");
+  }
+  if (x_dtype == ISHZ_DT_BF16 && M == 1 && !few) {  // the GEMV makes the row's image while staging x
+    const Out o{y, ISHZ_DT_BF16, nullptr};
+    switch (type) {
+#define X(T, F)                                                                                    \
+  case T:                                                                                          \
+    if (K % F::GEMV_K_MULT == 0) return gemv<F>(x, K, blocks, N, o, st);                           \
+    break;
+      ISHZ_GGML_FORMATS(X)
+#undef X
+    }
   }
   StreamTemp tmp(st);
   void *img = workspace;

@@ -196,26 +196,61 @@ struct GgmlGemv {
       }
     }
   }
-  static DEV void stage(const Args &, const uint16_t *x, u4 *xs, float *xsum, u4 *extra, int units,
-                        const XPre &pre) {
-    stage_body(x, xs, xsum, extra, units, pre);
+  template <class A>
+  static DEV void stage(const A &, const uint16_t *x, u4 *xs, float *xsum, u4 *extra, int units, XPre &pre,
+                        float down = 0.0f) {
+    stage_body(x, xs, xsum, extra, units, pre, down);
   }
-  // The staging itself (formats with their own Args call it from their stage).
-  static DEV void stage_body(const uint16_t *x, u4 *xs, float *xsum, u4 *extra, int units, const XPre &pre) {
+  // bf16 x: the exponent e of the row's largest magnitude (bf16_row_exponent), over the slots of every
+  // thread (those of the first round are in `pre`). scratch: one word per wave of the LDS that the
+  // staging fills afterwards. A launch that wrote the image first cost 10 us and more; the two
+  // barriers here cost about half a microsecond.
+  static DEV int bf16_scale(const uint16_t *x, int units, const XPre &pre, uint32_t *scratch) {
+    const int ns = (units + 15) / 16 * 16 * D::R, bd = blockDim.x;
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < U; j++) m = bf16_absmax(pre.v[j], m);
+    for (int i0 = threadIdx.x + U * bd; i0 < ns; i0 += U * bd) {
+      u4 v[U];
+      load_slots(x, units, i0, v);
+#pragma unroll
+      for (int j = 0; j < U; j++) m = bf16_absmax(v[j], m);
+    }
+    return bf16_row_exponent(block_absmax(m, scratch));
+  }
+  static DEV void half_slots(u4 *v, float down) {
+    if (down == 0.0f) return;
+#pragma unroll
+    for (int j = 0; j < U; j++) v[j] = bf16_to_half8(v[j], down);
+  }
+  static DEV void half_sums(u4 (*v)[SLMAX], float down) {
+    if (down == 0.0f) return;
+#pragma unroll
+    for (int j = 0; j < US; j++)
+#pragma unroll
+      for (int h = 0; h < D::SUM_LEN / 8; h++) v[j][h] = bf16_to_half8(v[j][h], down);
+  }
+  // The staging itself (formats with their own Args call it from their stage); down: see half_slots.
+  static DEV void stage_body(const uint16_t *x, u4 *xs, float *xsum, u4 *extra, int units, XPre &pre,
+                             float down = 0.0f) {
     const int ug = (units + 15) / 16, bd = blockDim.x;
     const int ns = ug * 16 * D::R;
+    half_slots(pre.v, down);
     store_slots(xs, units, threadIdx.x, pre.v);  // first round: loads issued by stage_load
     for (int i0 = threadIdx.x + U * bd; i0 < ns; i0 += U * bd) {
       u4 v[U];
       load_slots(x, units, i0, v);
+      half_slots(v, down);
       store_slots(xs, units, i0, v);
     }
     if constexpr (D::XSUM) {
       const int nq = ug * 16 * D::Q;
+      half_sums(pre.sv, down);
       store_sums(xsum, units, threadIdx.x, pre.sv);
       for (int i0 = threadIdx.x + US * bd; i0 < nq; i0 += US * bd) {
         u4 v[US][SLMAX];
         load_sums(x, units, i0, v);
+        half_sums(v, down);
         store_sums(xsum, units, i0, v);
       }
     }

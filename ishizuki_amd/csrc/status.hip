@@ -1,4 +1,5 @@
 // Status reporting of the C ABI: the reason for the calling thread's last non-OK status.
+#include <algorithm>
 #include <cstdio>
 
 #include "common.h"
@@ -23,54 +24,35 @@ int einval(const std::string &why) {
   return ISHZ_EINVAL;
 }
 
-// One workgroup per row: the row's largest magnitude (a max over the block), then every value
-// times 2^-e rounded to fp16.
-__global__ __launch_bounds__(256) void act_half_kernel(const void *__restrict__ x, int dt, int K,
-                                                       uint16_t *__restrict__ xh, float *__restrict__ rs) {
-  __shared__ float wmax[4];
-  const size_t row = (size_t)blockIdx.x * K;
-  // eight loads in flight per thread and pass (one at a time waited out a memory latency each)
-  constexpr int U = 8;
-  float m = 0.0f;
-  for (int k0 = threadIdx.x; k0 < K; k0 += U * blockDim.x) {
-    float v[U];
+// One workgroup per row: the row's largest magnitude, then every value times 2^-e rounded to fp16.
+// A row is a few tens of KB, so latency bounds it: every thread has its whole share of the row (up
+// to U 16-byte loads) in flight at once and keeps it in registers between the two passes. With one
+// 2-byte load per value and 256 threads, K = 5120 took 10 us and K = 25600 60 us.
+__global__ __launch_bounds__(1024) void act_half_kernel(const uint16_t *__restrict__ x, int K,
+                                                        uint16_t *__restrict__ xh, float *__restrict__ rs) {
+  __shared__ uint32_t wmax[16];
+  constexpr int U = 4;  // 1024 threads hold 32768 values; longer rows are read again by the second pass
+  const int n8 = K / 8, nt = blockDim.x;
+  const u4 *src = (const u4 *)(x + (size_t)blockIdx.x * K);
+  u4 *dst = (u4 *)(xh + (size_t)blockIdx.x * K);
+  u4 v[U];
+  auto load = [&](int i0) {
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int k = k0 + u * (int)blockDim.x;
-      v[u] = k < K ? fabsf(load_act(x, row + k, dt)) : 0.0f;
-    }
+    for (int u = 0; u < U; u++) v[u] = ld16<2>((const uint8_t *)(src + min(i0 + u * nt, n8 - 1)));
+  };
+  uint32_t m = 0;
+  for (int i0 = threadIdx.x; i0 < n8; i0 += U * nt) {
+    load(i0);
 #pragma unroll
-    for (int u = 0; u < U; u++) m = fmaxf(m, v[u]);
+    for (int u = 0; u < U; u++) m = bf16_absmax(v[u], m);
   }
-  m = fmaxf(m, ISHZ_DPP(m, 0xB1));   // the wave's max: quad, half-row and row by DPP,
-  m = fmaxf(m, ISHZ_DPP(m, 0x4E));
-  m = fmaxf(m, ISHZ_DPP(m, 0x141));
-  m = fmaxf(m, ISHZ_DPP(m, 0x140));
-  m = fmaxf(m, lane_xor16(m));       // across rows by the row swaps
-  m = fmaxf(m, lane_xor32(m));
-  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
-  __syncthreads();
-  m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-  // m = f 2^e, f in [0.5, 1), for every finite non-zero m; e capped at 127 so that 2^e stays a
-  // finite fp32 factor (a row whose largest value lies in (2^127, FLT_MAX] lands in [0.5, 2))
-  int e = 0;
-  if (m > 0.0f && __builtin_isfinite(m)) {
-    (void)frexpf(m, &e);
-    e = e > 127 ? 127 : e;
-  }
+  const int e = bf16_row_exponent(block_absmax(m, wmax));
   const float down = ldexpf(1.0f, -e);
-  for (int k0 = threadIdx.x; k0 < K; k0 += U * blockDim.x) {
-    float v[U];
+  for (int i0 = threadIdx.x; i0 < n8; i0 += U * nt) {
+    if (n8 > U * nt) load(i0);
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int k = k0 + u * (int)blockDim.x;
-      v[u] = k < K ? load_act(x, row + k, dt) : 0.0f;
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int k = k0 + u * (int)blockDim.x;
-      if (k < K) xh[row + k] = f2h(v[u] * down);
-    }
+    for (int u = 0; u < U; u++)
+      if (i0 + u * nt < n8) dst[i0 + u * nt] = bf16_to_half8(v[u], down);
   }
   if (threadIdx.x == 0) rs[blockIdx.x] = ldexpf(1.0f, e);
 }
@@ -84,11 +66,12 @@ int act_prepare(const void *x, int dt, int M, int K, void *image, hipStream_t st
     *rs = nullptr;
     return ISHZ_OK;
   }
-  if (dt != ISHZ_DT_BF16 && dt != ISHZ_DT_F32) return decline("activations must be fp16, bf16 or fp32");
-  if (!image) return einval("bf16 / fp32 activations need a workspace");
+  if (dt != ISHZ_DT_BF16 || K % 8) return decline("the fp16 image takes bf16 rows of a multiple of 8 values");
+  if (!image) return einval("bf16 activations need a workspace");
   uint16_t *h = (uint16_t *)image;
   float *r = (float *)((char *)image + ((size_t)M * K * 2 + 255) / 256 * 256);
-  hipLaunchKernelGGL(act_half_kernel, dim3(M), dim3(256), 0, st, x, dt, K, h, r);
+  const int nt = std::min(1024, (K / 8 + 63) / 64 * 64);
+  hipLaunchKernelGGL(act_half_kernel, dim3(M), dim3(nt), 0, st, (const uint16_t *)x, K, h, r);
   ISHZ_LAUNCH_CHECK("activation image launch");
   *xh = h;
   *rs = r;

@@ -196,3 +196,49 @@ def test_affine_rotated_linear_fp32(bits, M):
     ref = oracle.affine_matmul(xr, codes, s.view(np.uint16), b.view(np.uint16), N, bits, 64)
     W = oracle.affine_dequant(codes, s.view(np.uint16), b.view(np.uint16), N, K, bits, 64)
     check(y, ref, np.abs(xr) @ np.abs(W).T, torch.float32, f"affine linear fp32 bits={bits} M={M}")
+
+
+@pytest.mark.parametrize("scale", [1.0, 1.0e6, 1.0e-30])
+@pytest.mark.parametrize("t,M,K", [(ggml.Q4_K, 1, 256), (ggml.Q4_K, 1, 8448), (ggml.IQ2_XS, 1, 18176), (ggml.Q6_K, 1, 25600),
+                                   (ggml.Q4_0, 1, 32 * 7), (ggml.Q4_0, 1, 33024), (ggml.Q4_K, 2, 33024)])
+def test_bf16_row_image_edges(t, M, K, scale):
+    """The row's power-of-two factor found while the GEMV stages x (M = 1): rows within one staging
+    round and past it (256, 512 and 1024 threads hold 8192, 16384 and 32768 values), a K the GEMV does
+    not take, and the image launch beyond the 32768 values it keeps in registers (M = 2). The
+    largest value sits at the row's end."""
+    N = 40
+    blocks = synth.ggml_blocks(t, N, K, seed=t + K)
+    x = np.random.default_rng(K).standard_normal((M, K)).astype(np.float32)
+    x[:, -1] = 9.0
+    xt = torch.from_numpy(x * np.float32(scale)).to(torch.bfloat16)
+    print(f"bf16 row image t={t} M={M} K={K} scale={scale}", flush=True)
+    y = ggml.matvec(xt.to(DEV), torch.from_numpy(blocks).to(DEV), t, N)
+    ref, bd = ggml_reference(t, xt.float().numpy(), blocks, N)
+    check(y, ref, bd, torch.bfloat16, f"bf16 image t={t} K={K}")
+
+
+@pytest.mark.parametrize("bits,K", [(2, 128), (2, 16896), (4, 8448)])
+def test_bf16_row_image_edges_affine(bits, K):
+    N = 40
+    codes, s, b = (synth.affine_pack if bits == 2 else lambda *a, **k: synth.affine_pack_bits(*a, bits, **k))(
+        N, K, group=64, seed=bits)
+    x = np.random.default_rng(K).standard_normal((1, K)).astype(np.float32)
+    x[0, -1] = 9.0
+    xt = torch.from_numpy(x).to(torch.bfloat16)
+    dev = [torch.from_numpy(a).to(DEV) for a in (codes.view(np.int32), s, b)]
+    y = affine.quantized_matmul(xt.to(DEV), *dev, group_size=64, bits=bits)
+    xf = xt.float().numpy()
+    ref = oracle.affine_matmul(xf, codes, s.view(np.uint16), b.view(np.uint16), N, bits, 64)
+    W = oracle.affine_dequant(codes, s.view(np.uint16), b.view(np.uint16), N, K, bits, 64)
+    check(y, ref, np.abs(xf) @ np.abs(W).T, torch.bfloat16, f"affine bf16 image bits={bits} K={K}")
+
+
+def test_bf16_row_image_non_finite():
+    """A row with an infinity or a NaN gives no finite output; a row of zeros gives zeros."""
+    N, K = 40, 512
+    blk = torch.from_numpy(synth.ggml_blocks(ggml.Q4_K, N, K, seed=3)).to(DEV)
+    for v in (float("inf"), float("nan")):
+        x = torch.ones(1, K, dtype=torch.bfloat16, device=DEV)
+        x[0, 7] = v
+        assert not torch.isfinite(ggml.matvec(x, blk, ggml.Q4_K, N)).any()
+    assert (ggml.matvec(torch.zeros(1, K, dtype=torch.bfloat16, device=DEV), blk, ggml.Q4_K, N) == 0).all()
