@@ -146,6 +146,16 @@ int ishz_affine_linear(const void *x, int x_dtype, int M, int K, const float *si
                        int scale_dtype, int N, int bits, int group, void *y, void *workspace,
                        size_t workspace_bytes, ishz_stream_t stream);
 
+/* ishz_affine_linear for prompts: any number of rows in one call (the reference runs prompts through
+   MLX's quantizedMM). fp16 or bf16 x, packs of 2, 4, 6 and 8 bits in groups of 64 or 128, K a
+   multiple of 256; declines the rest, which go to ishz_affine_linear 16 rows at a time. The same
+   exact codes, fp32 scales and fp32 sums. */
+size_t ishz_affine_rows_workspace_size(int M, int K, int N);
+int ishz_affine_linear_rows(const void *x, int x_dtype, int M, int K, const float *signs, int block,
+                            const uint32_t *codes, const void *scales, const void *biases,
+                            int scale_dtype, int N, int bits, int group, void *y, void *workspace,
+                            size_t workspace_bytes, ishz_stream_t stream);
+
 /* EXL3 codebooks (EXL3Tensor.Codebook, Core/EXL3.swift:10-14); rates are bits2 = 2 * bits in
    {2,3,4,5,6,7,8,10,12,14,16} (supportedBits, :27), half-integer rates only with MUL1. */
 enum { ISHZ_EXL3_3INST = 0, ISHZ_EXL3_MCG = 1, ISHZ_EXL3_MUL1 = 2 };
@@ -185,6 +195,13 @@ size_t ishz_exl3_workspace_size(int M, int K, int N);
 int ishz_exl3_apply(const void *x, int x_dtype, int M, int K, const int16_t *trellis,
                     const uint16_t *suh, const uint16_t *svh, int N, int bits2, int codebook,
                     void *y, void *workspace, size_t workspace_bytes, ishz_stream_t stream);
+
+/* ishz_exl3_apply for prompts: any number of rows in one call. fp16 or bf16 x, K a multiple of 256;
+   declines the rest. Every weight is decoded to its exact fp16 value. */
+size_t ishz_exl3_rows_workspace_size(int M, int K, int N);
+int ishz_exl3_apply_rows(const void *x, int x_dtype, int M, int K, const int16_t *trellis,
+                         const uint16_t *suh, const uint16_t *svh, int N, int bits2, int codebook,
+                         void *y, void *workspace, size_t workspace_bytes, ishz_stream_t stream);
 
 /* No counterpart in the reference: ishz_exl3_apply for callers that cannot allocate (code under
    HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). It allocates nothing:

@@ -30,6 +30,10 @@ _SIGS = {
     "ishz_affine_matmul": (I, [P, I, I, I, P, P, P, I, I, I, I, P, P]),
     "ishz_affine_workspace_size": (SZ, [I, I]),
     "ishz_affine_linear": (I, [P, I, I, I, P, I, P, P, P, I, I, I, I, P, P, SZ, P]),
+    "ishz_affine_rows_workspace_size": (SZ, [I, I, I]),
+    "ishz_affine_linear_rows": (I, [P, I, I, I, P, I, P, P, P, I, I, I, I, P, P, SZ, P]),
+    "ishz_exl3_rows_workspace_size": (SZ, [I, I, I]),
+    "ishz_exl3_apply_rows": (I, [P, I, I, I, P, P, P, I, I, I, P, P, SZ, P]),
     "ishz_exl3_dequant": (I, [P, I, I, I, I, P, I, P]),
     "ishz_exl3_rotate": (I, [P, I, I, I, P, I, P, I, P]),
     "ishz_exl3_matvec": (I, [P, I, I, I, P, I, I, I, P, P]),

@@ -85,3 +85,22 @@ def linear(x, weight, scales, biases, signs=None, block=0, group_size=64, bits=2
     rc = L.ishz_affine_linear(ptr(x), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, w, sc, b, sdt, N,
                               bits, group_size, ptr(y), ptr(ws), ws_bytes, stream())
     return y if _lib.check(rc, "affine_linear") else None
+
+
+def linear_rows(x, weight, scales, biases, signs=None, block=0, group_size=64, bits=2):
+    """The rotated PackedLinear forward for a prompt: any number of rows in one call; None if
+    declined (fp32 x, odd widths, other groups), where `linear` takes 16 rows at a time."""
+    require_cuda(x, weight, scales, biases)
+    x = x.contiguous()
+    M, K = x.shape
+    N = weight.shape[0]
+    L = _lib.lib()
+    ws = torch.empty(L.ishz_affine_rows_workspace_size(M, K, N), dtype=torch.uint8, device=x.device)
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    s = None
+    if block and signs is not None:
+        s = signs.to(device=x.device, dtype=torch.float32).contiguous()
+    w, sc, b, sdt = _args(weight, scales, biases)
+    rc = L.ishz_affine_linear_rows(ptr(x), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, w, sc, b, sdt, N, bits,
+                                   group_size, ptr(y), ptr(ws), ws.numel(), stream())
+    return y if _lib.check(rc, "affine_linear_rows") else None

@@ -19,57 +19,12 @@
 #include <string>
 
 #include "common.h"
-
+#include "exl3_fmt.h"
+#include "qgemm.h"
 
 namespace ishz {
-
-// exl3_decode (EXL3.swift:136-147): 3INST / MCG / MUL1 codebooks, fp16 single rounding.
-DEV _Float16 exl3_decode(uint32_t s, int cb) {
-  if (cb == 2) {
-    const uint32_t x = s * 0x83DCD12Du;
-    const uint32_t p = (x & 0x00ff00ffu) + ((x >> 8) & 0x00ff00ffu);
-    const _Float16 h = __builtin_bit_cast(_Float16, (uint16_t)((p & 0xffffu) + (p >> 16) + 0x6400u));
-    return __builtin_fmaf16(h, __builtin_bit_cast(_Float16, (uint16_t)0x1eee),
-                            __builtin_bit_cast(_Float16, (uint16_t)0xc931));
-  }
-  uint32_t x = cb == 1 ? s * 0xCBAC1FEDu : s * 89226354u + 64248484u;
-  x = (x & 0x8fff8fffu) ^ 0x3b603b60u;
-  return __builtin_bit_cast(_Float16, (uint16_t)x) + __builtin_bit_cast(_Float16, (uint16_t)(x >> 16));
-}
-
-// Where the states lie in a tile's bit ring. At an integer rate of KA bits per weight, position p
-// consumes KA bits and its state ends at ring bit KA (p + 1). At a half rate (KA + 1/2 bits) an
-// even/odd pair consumes 2 KA + 1 bits, the even position KA of them and the odd one KA + 1. A
-// state is the 16 ring bits ending there, read MSB first (bit 0 is the top bit of word 0), so it
-// reaches back into the bits of earlier positions and wraps around the ring.
-template <int KA, bool HALF>
-struct Trellis {
-  static constexpr int RING = HALF ? 128 * (2 * KA + 1) : 256 * KA;  // bits per 16x16 tile
-  static constexpr int WORDS = RING / 32;
-  static __host__ __device__ constexpr int bit_end(int p) {
-    return HALF ? (p / 2) * (2 * KA + 1) + KA + (p % 2) * (KA + 1) : (p + 1) * KA;
-  }
-  // First ring bit of position p's state.
-  static DEV int first_bit(int p) { return (bit_end(p) + RING - 16) % RING; }
-  // Start of the state of position p0 + i relative to that of p0 (p0 even).
-  static constexpr int offset(int i) { return bit_end(i) - bit_end(0); }
-  // The 16-bit state starting at ring bit b: the 32 bits from b are one funnel shift of the word
-  // holding b and the next word (b on a word boundary: that word alone); the state is the top half.
-  static DEV uint32_t state(const uint32_t *tile, int b) {
-    const int w = b >> 5, o = b & 31;
-    const uint32_t hi = tile[w];
-    const uint32_t bits32 = o ? __builtin_amdgcn_alignbit(hi, tile[(w + 1) % WORDS], 32 - o) : hi;
-    return bits32 >> 16;
-  }
-  // The four weights at positions p0 .. p0 + 3, as two packed fp16 pairs.
-  static DEV u2 decode4(const uint32_t *tile, int p0, int cb) {
-    uint32_t h[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-      h[i] = __builtin_bit_cast(uint16_t, exl3_decode(state(tile, (first_bit(p0) + offset(i)) % RING), cb));
-    return u2{h[0] | h[1] << 16, h[2] | h[3] << 16};
-  }
-};
+int exl3_rows_core(const void *xr, int dt, int M, int K, const int16_t *trellis, int N, int bits2, int cb, void *ws, float *part,
+                   int S, const float **rs, hipStream_t st);
 
 // ------------------------------------------------------------------- matvec / verify
 // A workgroup owns one column tile tn (16 outputs); its KS waves take tiles tk = wave, wave+KS,
@@ -186,59 +141,10 @@ __global__ __launch_bounds__(256) void exl3_mm_f32(const float *__restrict__ x, 
 // two tile words, each state one bit-field extract, and two weights are decoded per packed fp16
 // operation. A workgroup owns TN column tiles and its waves split the K tiles (tk = wave, wave +
 // KS, ...), keeping D steps of tile words and x in flight; partials meet in LDS at the end.
-template <int KA, bool HALF>
-struct Trellis32 {
-  using TR = Trellis<KA, HALF>;
-  static constexpr bool FITS = TR::offset(3) <= 16;  // the four states within 32 bits
-  // The lane's 32-bit window (from the first bit of p0's state): words ja, jb funnel-shifted by amt.
-  struct Win {
-    int ja, jb, amt;
-  };
-  static DEV Win window(int p0) {
-    const int b = TR::first_bit(p0), w = b >> 5, o = b & 31;
-    return o ? Win{w, (w + 1) % TR::WORDS, 32 - o} : Win{w, w, 0};
-  }
-  // Bit-field offset of state i inside the window.
-  static constexpr int field(int i) { return 16 - TR::offset(i); }
-};
-
-// Codebook images of two states, packed as fp16 (a in the low half): exl3_decode, pairwise.
-template <int CB>
-DEV uint32_t exl3_decode2(uint32_t sa, uint32_t sb) {
-  if constexpr (CB == 2) {
-    auto p = [](uint32_t s) {
-      const uint32_t x = s * 0x83DCD12Du;
-      const uint32_t q = (x & 0x00ff00ffu) + ((x >> 8) & 0x00ff00ffu);
-      return ((q & 0xffffu) + (q >> 16) + 0x6400u) & 0xffffu;
-    };
-    const h2 h = as_h2(p(sa) | p(sb) << 16);
-    const h2 m = as_h2(0x1eee1eeeu), c = as_h2(0xc931c931u);
-    return __builtin_bit_cast(uint32_t, (h2)__builtin_elementwise_fma(h, m, c));
-  } else {
-    auto x = [](uint32_t s) {
-      const uint32_t v = CB == 1 ? s * 0xCBAC1FEDu : s * 89226354u + 64248484u;
-      return (v & 0x8fff8fffu) ^ 0x3b603b60u;
-    };
-    const uint32_t xa = x(sa), xb = x(sb);
-    const uint32_t lo = __builtin_amdgcn_perm(xb, xa, 0x05040100u), hi = __builtin_amdgcn_perm(xb, xa, 0x07060302u);
-    return __builtin_bit_cast(uint32_t, as_h2(lo) + as_h2(hi));
-  }
-}
-
-// 3INST / MCG image of one state as the two fp16 halves whose sum is the weight (exl3_decode
-// before its final add). The M = 1 matvec multiplies them by (x, x) as two MFMA k-entries: the
-// halves meet x in fp32, so the weight's fp16 rounding of their sum is skipped (a difference of
-// at most half an fp16 ulp per weight, inside the matmul tolerance; dequantization keeps the
-// exact decode).
-template <int CB>
-DEV uint32_t exl3_halves(uint32_t s) {
-  static_assert(CB != 2, "MUL1 decodes to one fp16 directly");
-  const uint32_t v = CB == 1 ? s * 0xCBAC1FEDu : s * 89226354u + 64248484u;
-  return (v & 0x8fff8fffu) ^ 0x3b603b60u;
-}
-DEV uint32_t dup_lo(uint32_t p) { return __builtin_amdgcn_perm(p, p, 0x01000100u); }
-DEV uint32_t dup_hi(uint32_t p) { return __builtin_amdgcn_perm(p, p, 0x03020302u); }
-
+// ------------------------------------------------------------------- streaming matvec / verify
+// For rates whose four lane states span at most 32 bits (Trellis32). A workgroup owns TN column tiles and
+// its waves split the K tiles (tk = wave, wave + KS, ...), keeping D steps of tile words and x in
+// flight; partials meet in LDS at the end.
 template <int KA, bool HALF, int CB, bool MF, int TN, int D>
 __global__ __launch_bounds__(1024) void exl3_mm2(const uint16_t *__restrict__ xh, int M, int K,
                                                 const uint32_t *__restrict__ trellis, int N,
@@ -978,6 +884,39 @@ extern "C" int ishz_exl3_apply(const void *x, int x_dtype, int M, int K, const i
   const size_t blocks = (size_t)M * (N / 128);  // output rotation, summing the K-split partials
   hipLaunchKernelGGL(exl3_rotate_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, st, yh,
                      ISHZ_DT_F32, blocks, N, svh, 0, y, x_dtype, np, rs);
+  ISHZ_LAUNCH_CHECK("exl3 rotate launch");
+  return ISHZ_OK;
+}
+
+// ishz_exl3_apply for any number of rows (fp16 / bf16, K a multiple of 256). Workspace: x rotated in its
+// own dtype, the many-row kernel's image, then the K parts' products, which the output rotation sums.
+extern "C" size_t ishz_exl3_rows_workspace_size(int M, int K, int N) {
+  if (M <= 0 || K <= 0 || N <= 0 || K % 256) return 0;
+  const int S = qgemm_splits(M, K, N, qgemm_mt(8, M), num_cu_e());
+  return q256((size_t)M * K * 2) + qgemm_layout(M, K, N, 0, qgemm_mt(8, M)).part + (size_t)S * M * N * 4;
+}
+
+extern "C" int ishz_exl3_apply_rows(const void *x, int x_dtype, int M, int K, const int16_t *trellis, const uint16_t *suh,
+                                    const uint16_t *svh, int N, int bits2, int codebook, void *y, void *workspace,
+                                    size_t workspace_bytes, ishz_stream_t stream) {
+  int rc = check_exl3(K, N, bits2, codebook);
+  if (rc) return rc;
+  if (x_dtype != ISHZ_DT_F16 && x_dtype != ISHZ_DT_BF16) return decline("many rows: activations must be fp16 or bf16");
+  if (M < 1 || K % 256) return decline("many rows: K a multiple of 256");
+  if ((rc = by_rate(bits2, []<int KA, bool HALF>() -> int { return ISHZ_OK; }))) return rc;
+  if (!x || !trellis || !suh || !svh || !y) return einval("null pointer");
+  if (!workspace || workspace_bytes < ishz_exl3_rows_workspace_size(M, K, N))
+    return einval("workspace too small (ishz_exl3_rows_workspace_size)");
+  hipStream_t st = S(stream);
+  const int parts = qgemm_splits(M, K, N, qgemm_mt(8, M), num_cu_e());
+  uint8_t *xr = (uint8_t *)workspace, *ws = xr + q256((size_t)M * K * 2);
+  float *yh = (float *)(ws + qgemm_layout(M, K, N, 0, qgemm_mt(8, M)).part);
+  if ((rc = ishz_exl3_rotate(x, x_dtype, M, K, suh, 1, xr, x_dtype, stream))) return rc;
+  const float *rs;
+  if ((rc = exl3_rows_core(xr, x_dtype, M, K, trellis, N, bits2, codebook, ws, yh, parts, &rs, st))) return rc;
+  const size_t blocks = (size_t)M * (N / 128);
+  hipLaunchKernelGGL(exl3_rotate_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, st, yh, ISHZ_DT_F32, blocks, N, svh, 0,
+                     y, x_dtype, parts, rs);
   ISHZ_LAUNCH_CHECK("exl3 rotate launch");
   return ISHZ_OK;
 }

@@ -89,3 +89,17 @@ def apply(x, t):
     if not _lib.check(rc, "exl3_apply"):
         return None
     return y.reshape(*shape[:-1], t.output_dim)
+
+
+def apply_rows(x, t):
+    """EXL3Kernels.apply for a prompt: any number of rows [M, K] in one call; None if declined (fp32 x,
+    K not a multiple of 256), where `apply` takes 16 rows at a time."""
+    require_cuda(x, t.trellis)
+    x = x.contiguous()
+    M = x.shape[0]
+    L = _lib.lib()
+    ws = torch.empty(L.ishz_exl3_rows_workspace_size(M, t.input_dim, t.output_dim), dtype=torch.uint8, device=x.device)
+    y = torch.empty((M, t.output_dim), dtype=x.dtype, device=x.device)
+    rc = L.ishz_exl3_apply_rows(ptr(x), DTYPES.get(x.dtype, -1), M, t.input_dim, ptr(t.trellis), ptr(t.suh), ptr(t.svh),
+                                t.output_dim, t.bits2, t.codebook, ptr(y), ptr(ws), ws.numel(), stream())
+    return y if _lib.check(rc, "exl3_apply_rows") else None

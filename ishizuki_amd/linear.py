@@ -8,8 +8,10 @@ that dispatches as `callAsFunction` (:180-231) does:
 * EXL3 -> `exl3.apply` (EXL3Kernels.apply);
 * dense fp16 -> `x @ W^T`;
 * MLX affine pack (2, 4 or 8 bits), rotated by a blockwise Hadamard transform when `block` > 0
-  -> `affine.linear` (rotation fused for blocks up to 128, then the quantized matmul), in calls
-  of at most 16 rows.
+  -> `affine.linear` (rotation fused for blocks up to 128, then the quantized matmul).
+
+More than 16 rows of an EXL3 tensor or an affine pack are one call of the many-row kernels where they
+take it, else calls of 16 rows.
 
 The forward returns None where the reference's kernels return nil (a declined shape or dtype).
 """
@@ -71,6 +73,9 @@ class PackedLinear:
         if self.exl3 is not None:
             shape = x.shape
             rows = x.reshape(-1, shape[-1])
+            y = exl3.apply_rows(rows, self.exl3) if rows.shape[0] > 16 else None
+            if y is not None:
+                return y.reshape(*shape[:-1], self.output_dim)
             parts = [exl3.apply(rows[r:r + 16], self.exl3) for r in range(0, rows.shape[0], 16)]
             if any(p is None for p in parts):
                 return None
@@ -80,6 +85,11 @@ class PackedLinear:
         shape = x.shape
         rows = x.reshape(-1, shape[-1])
         signs = self.signs if self.block > 0 else None
+        if rows.shape[0] > 16:
+            y = affine.linear_rows(rows, self.weight, self.scales, self.biases, signs=signs, block=self.block,
+                                   group_size=self.group_size, bits=self.bits)
+            if y is not None:
+                return y.reshape(*shape[:-1], self.output_dim)
         parts = [affine.linear(rows[r:r + 16], self.weight, self.scales, self.biases, signs=signs, block=self.block,
                                group_size=self.group_size, bits=self.bits) for r in range(0, rows.shape[0], 16)]
         if any(p is None for p in parts):
