@@ -8,38 +8,10 @@
 
 #define ISHZ_TABLE_QUAL static __device__
 #include "ggml_grids.inc"
+#include "ggml_tables.h"
 #include "ggml_iq.h"
 
 namespace ishz {
-
-// ----------------------------------------------------------------------------- tables in LDS
-// IQ2_XS grid entries as fp16 (values 8, 25, 43), either in the permuted pair order of the GEMV
-// (x0,x2,x1,x3,...) or in natural order for the MFMA B operand; with `sgn`, also the 128 sign
-// patterns of ksigns (index | parity << 7) as natural-order fp16 sign-bit masks (the GEMV computes
-// its masks in registers).
-template <bool PERM>
-DEV void build_iq2xs_tables(u4 *grid, u4 *sgn) {
-  for (int e = threadIdx.x; e < 512 + (sgn ? 128 : 0); e += blockDim.x) {
-    if (e < 512) {
-      const uint64_t v = ishz_iq2xs_grid[e];
-      uint32_t hv[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++) hv[j] = f2h((float)((v >> (8 * j)) & 0xff));
-      grid[e] = PERM ? u4{hv[0] | hv[2] << 16, hv[1] | hv[3] << 16, hv[4] | hv[6] << 16,
-                          hv[5] | hv[7] << 16}
-                     : u4{hv[0] | hv[1] << 16, hv[2] | hv[3] << 16, hv[4] | hv[5] << 16,
-                          hv[6] | hv[7] << 16};
-    } else {
-      const int i = e - 512;
-      const uint32_t s = (uint32_t)i | (uint32_t)(__builtin_popcount(i) & 1) << 7;
-      auto bit = [&](int j) { return ((s >> j) & 1u) << 15; };
-      sgn[i] = u4{bit(0) | bit(1) << 16, bit(2) | bit(3) << 16, bit(4) | bit(5) << 16, bit(6) | bit(7) << 16};
-    }
-  }
-}
-
-DEV void build_iq2xs_tables_perm(u4 *grid, u4 *sgn) { build_iq2xs_tables<true>(grid, sgn); }
-DEV void build_iq2xs_tables_nat(u4 *grid, u4 *sgn) { build_iq2xs_tables<false>(grid, sgn); }
 
 // ----------------------------------------------------------------------------- verify (MFMA)
 // A workgroup owns T tiles of 16 weight rows; its KS waves split the row's blocks round-robin
@@ -378,6 +350,12 @@ __global__ __launch_bounds__(256) void vgemm_sum_kernel(const float *__restrict_
   }
 }
 
+// Sixteen rows per MFMA (wgemm.hip).
+bool ggml_wgemm_takes(uint32_t type, int M, int K);
+size_t ggml_wgemm_part_bytes(int M, int K, int N, int cus);
+int ggml_wgemm(uint32_t type, const void *x, int M, int K, const void *w, int N, const Out &y, void *ws, size_t ws_bytes,
+               hipStream_t st);
+
 static int check_matmul(uint32_t type, int x_dtype, int M, int lo, int hi, int K,
                         size_t blocks_bytes, int N, const void *x, const void *w, const void *y) {
   const int bs = block_size(type);
@@ -402,6 +380,7 @@ extern "C" int ishz_ggml_type_size(uint32_t type) { return type_size(type); }
 // Workspace: the activation image (bf16 / fp32 x), then the K split's fp32 parts.
 extern "C" size_t ishz_ggml_workspace_size(uint32_t type, int M, int K, int N) {
   if (!block_size(type) || M < 1 || M > 16 || K <= 0 || N <= 0) return 0;
+  if (ggml_wgemm_takes(type, M, K)) return act_image_bytes(M, K) + ggml_wgemm_part_bytes(M, K, N, num_cu());
   return act_image_bytes(M, K) + (K % 256 ? 0 : vgemm_workspace(M, K, N, num_cu()));
 }
 
@@ -462,6 +441,7 @@ static int ggml_call(uint32_t type, const void *x, int x_dtype, int M, int K, co
     case ISHZ_GGML_IQ2_XS: return gemv<FIQ2_XS>(xh, K, blocks, N, o, st);
     }
   }
+  if (ggml_wgemm_takes(type, M, K)) return ggml_wgemm(type, xh, M, K, blocks, N, o, ws, wb, st);
   switch (type) {
   case ISHZ_GGML_Q4_0: return verify<FQ4_0>(xh, M, K, blocks, N, o, st, ws, wb);
   case ISHZ_GGML_Q4_K: return verify<FQ4_K>(xh, M, K, blocks, N, o, st, ws, wb);

@@ -211,3 +211,26 @@ def test_verify_k_split_matches_unsplit(t, M):
     ref, bd = ggml_reference(t, x.astype(np.float32), blocks, N)
     for y, what in zip(ys, ("split", "unsplit")):
         assert_close(y, ref, bound=bd, what=f"{what} t={t} M={M}")
+
+
+@pytest.mark.parametrize("t", [ggml.Q4_K, ggml.Q6_K, ggml.IQ2_XS])
+@pytest.mark.parametrize("M,N,K", [(5, 16, 256), (16, 17, 512), (9, 4100, 768), (16, 2050, 6144), (13, 100, 12544), (8, 33, 25600)])
+@pytest.mark.parametrize("workspace", [True, False])
+def test_sixteen_rows_per_mfma(t, M, N, K, workspace):
+    """The kernel for 5..16 rows: one tile, ragged last tiles, more tiles than one per CU, x in one and in
+    several chunks of K, K split into parts (with a workspace) and not. Sub-scales of both signs and every
+    nibble occur (uniform bytes); the products are exact, so the bound is that of the fp32 sums."""
+    from ishizuki_amd import _lib
+    from ishizuki_amd._torch import ptr, stream
+    L = _lib.lib()
+    blk = synth.ggml_blocks(t, N, K, seed=t + M + K)
+    x = synth.fp16_normal((M, K), seed=M)
+    print(f"16 rows per MFMA t={t} M={M} N={N} K={K} workspace={workspace}", flush=True)
+    xd, bd = torch.from_numpy(x).to(DEV), torch.from_numpy(blk).to(DEV)
+    y = torch.empty((M, N), dtype=torch.float16, device=DEV)
+    wsb = L.ishz_ggml_workspace_size(t, M, K, N) if workspace else 0
+    ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=DEV)
+    rc = L.ishz_ggml_matvec_ws(t, ptr(xd), 1, M, K, ptr(bd), blk.nbytes, N, ptr(y), ptr(ws) if wsb else None, wsb, stream())
+    assert rc == _lib.OK, _lib.last_error()
+    ref, bound = ggml_reference(t, x.astype(np.float32), blk, N)
+    assert_close(y.float().cpu().numpy(), ref, bound=bound, what=f"t={t} M={M} N={N} K={K}")
