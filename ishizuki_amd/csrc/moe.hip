@@ -26,7 +26,9 @@
 
 #include "affine_nbit.h"
 #include "ggml_formats.h"
+#include "qgemm.h"
 #include "vgemm.h"
+#include "wgemm.h"
 
 namespace ishz {
 
@@ -382,27 +384,58 @@ __global__ __launch_bounds__(1024) void moe_down_kernel(const uint16_t *__restri
   }
 }
 
+// W outputs of a token per thread: eight (one 16-byte load per slot; H is a multiple of 32) once that
+// still fills the chip, one for few tokens (T = 8: eight a thread took 1 us longer).
+template <int W>
 static __global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t *__restrict__ o, int H,
                                                           int T, int k, MoeRoute R,
                                                           const uint16_t *__restrict__ shared,
                                                           const uint16_t *__restrict__ shared_gate,
                                                           uint16_t *__restrict__ y, bool bf) {
-  const size_t total = (size_t)T * H;
+  const size_t hn = H / W, total = (size_t)T * hn;
+  struct Val {
+    uint16_t v[W];
+  };
+  auto ld = [](const uint16_t *p) {
+    Val r;
+    __builtin_memcpy(&r, __builtin_assume_aligned(p, 2), sizeof(r));
+    return r;
+  };
   by_act(bf, [&]<bool BF>() {
     for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < total;
          q += (size_t)gridDim.x * blockDim.x) {
-      const int t = (int)(q / H), n = (int)(q % H);
-      float acc = 0.0f;
+      const int t = (int)(q / hn), n = (int)(q % hn) * W;
+      float acc[W] = {};
       for (int s = 0; s < k; s++) {
-        acc += from16<BF>(o[((size_t)t * k + s) * H + n]) * R.w[t * k + s];  // o rows in slot order
+        const Val v = ld(o + ((size_t)t * k + s) * H + n);  // o rows in slot order
+        const float w = R.w[t * k + s];
+#pragma unroll
+        for (int e = 0; e < W; e++) acc[e] += from16<BF>(v.v[e]) * w;
       }
       if (shared) {  // the shared expert, widened and added before the one narrowing
         const float sg = rnd<BF>(1.0f / (1.0f + __expf(-from16<BF>(shared_gate[t]))));
-        acc += rnd<BF>(sg * from16<BF>(shared[q]));
+        const Val v = ld(shared + q * W);
+#pragma unroll
+        for (int e = 0; e < W; e++) acc[e] += rnd<BF>(sg * from16<BF>(v.v[e]));
       }
-      y[q] = bits16<BF>(acc);
+      Val r;
+#pragma unroll
+      for (int e = 0; e < W; e++) r.v[e] = bits16<BF>(acc[e]);
+      __builtin_memcpy(__builtin_assume_aligned(y + q * W, 2), &r, sizeof(r));
     }
   });
+}
+static int moe_combine(const uint16_t *o, int H, int T, int k, const MoeRoute &R, const uint16_t *shared,
+                       const uint16_t *shared_gate, void *y, bool bf, hipStream_t st) {
+  const size_t total = (size_t)T * H;
+  auto launch = [&](auto kern, size_t n) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, st, o, H, T, k, R, shared,
+                       shared_gate, (uint16_t *)y, bf);
+  };
+  if (total >= (size_t)8 * 256 * 256) launch(moe_combine_kernel<8>, total / 8);
+  else launch(moe_combine_kernel<1>, total);
+  ISHZ_LAUNCH_CHECK("moe combine launch");
+  return ISHZ_OK;
 }
 
 // ------------------------------------------------------------------- streaming (MFMA) FFN
@@ -772,8 +805,25 @@ struct FMoeDown : F {
 
 // Quads per pass sized for about twice an expert's expected load (T k / E tokens) plus two;
 // an expert with more tokens takes further passes.
+// More than four tokens an expert on average: sixteen rows per MFMA (wgemm.h) for the formats it takes.
+template <class F>
+struct WOf {
+  static constexpr bool HAS = false;
+};
+template <>
+struct WOf<FQ4_K> {
+  static constexpr bool HAS = true;
+  using type = WQ4_K;
+};
+template <>
+struct WOf<FQ6_K> {
+  static constexpr bool HAS = true;
+  using type = WQ6_K;
+};
 template <class F, class P>
 static int moe_vgemm(const P &p, int T, int E, int k, int K, int rows, int groups, int tiles_per_wg, hipStream_t st) {
+  if constexpr (WOf<F>::HAS && !requires { p.prologue(); })
+    if (T * k > 4 * E) return launch_wgemm<typename WOf<F>::type>(p, 16, K, rows, groups, tiles_per_wg, 1, st);
   const int want = (2 * T * k / std::max(E, 1) + 2 + 3) / 4;
   switch (std::max(1, std::min({4, (T + 3) / 4, want}))) {
     case 1: return launch_vgemm_p<F, P, 1>(p, K, rows, groups, tiles_per_wg, st);
@@ -851,7 +901,8 @@ static bool route_in_gate_up(int T, int H, int E, int I, int k) {
 struct MoeAct {
   bool bf;
   const float *rsx;  // x's row factors (bf16), or null
-  void *himg;        // workspace for h's image (bf16)
+  void *himg;        // workspace for h's image (bf16, and the many-row kernel)
+  void *ximg;        // and for x's
 };
 // h's fp16 image and row factors for the down projection (bf16), or h itself.
 static int moe_h_image(const MoeAct &ma, const uint16_t *h, int P, int I, hipStream_t st, const uint16_t **h16,
@@ -872,7 +923,6 @@ static int moe_ffn(const void *x, int T, int H, int E, int I, int k, const void 
   const uint16_t *h16;
   const float *rsh;
   const int amax = std::min(E, T * k);
-  const size_t total = (size_t)T * H;
   // one or two tokens: every (token, slot) pair is a GEMV; two launches of the streaming GEMV
   // (routing in the first, the combine in the second)
   if (gathered_gemv(T, H, I, k)) {
@@ -932,10 +982,7 @@ static int moe_ffn(const void *x, int T, int H, int E, int I, int k, const void 
                        st, h16, I, (const uint8_t *)down, H, R, o, rsh, ma.bf);
     ISHZ_LAUNCH_CHECK("moe down launch");
   }
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)std::min<size_t>((total + 255) / 256, 4096)), dim3(256), 0,
-                     st, o, H, T, k, R, shared, shared_gate, (uint16_t *)y, ma.bf);
-  ISHZ_LAUNCH_CHECK("moe combine launch");
-  return ISHZ_OK;
+  return moe_combine(o, H, T, k, R, shared, shared_gate, y, ma.bf, st);
 }
 
 // Routing, and the pair lists when `place` (the streaming MFMA projections need them; the
@@ -945,7 +992,8 @@ static int moe_route_all(const float *logits, int T, int E, int topk, int normal
   const int nr = std::min((T + 3) / 4 * 4, 64);  // routing rows: whole waves, at most 16
   const size_t fused_lds = ((size_t)nr * route_row_words(E, topk) + E + (size_t)T * topk) * 4;
   if (!place) return route_launch(logits, T, E, topk, normalize, R, st);
-  if (fused_lds <= 64 * 1024) {
+  // (one workgroup routes 64 tokens at a time, about 4 us a round; 512 tokens took 56 us)
+  if (T <= 64 && fused_lds <= 64 * 1024) {
     hipLaunchKernelGGL(moe_route_place_kernel, dim3(1), dim3(16 * nr), fused_lds, st, logits, T, E, topk, normalize, R);
     ISHZ_LAUNCH_CHECK("moe route launch");
     return ISHZ_OK;
@@ -1010,6 +1058,73 @@ struct FMoeDownA : FMoeDown<F> {
   }
 };
 
+// Many tokens per expert: the many-row kernel (qgemm.h), one group per active expert. Gate and up rows
+// interleave by tile as above, so a wave's two column tiles are a SwiGLU pair.
+struct QMoeGateUpRows {
+  AffPack g;
+  int64_t dc, ds, db;  // bytes from gate's arrays to up's (a select between two packs would put them in scratch memory)
+  int e, I;
+  template <class T>
+  static DEV const T *at(const T *p, int64_t d) {
+    return (const T *)((const char *)p + d);
+  }
+  DEV AffRow arow(int row) const {
+    const int tile = row >> 4, i = min((tile >> 1) * 16 + (row & 15), I - 1);
+    const int64_t up = -(int64_t)(tile & 1);
+    const AffRow r = g.row((size_t)e * I + i);
+    return {at(r.codes, dc & up), at(r.scales, ds & up), at(r.biases, db & up)};
+  }
+};
+struct QMoeDownRows {
+  AffPack d;
+  int e, H;
+  DEV AffRow arow(int row) const { return d.row((size_t)e * H + row); }
+};
+struct QMoeGateUp : VMoeGateUp {
+  static constexpr bool RAGGED = true;
+  AffPack g, u;
+  DEV size_t src(const Group &gp, int i) const { return R.pair_q[gp.p0 + i] / k; }
+  DEV QMoeGateUpRows weights(const Group &gp) const {
+    auto diff = [](const void *a, const void *b) { return (int64_t)((const char *)b - (const char *)a); };
+    return {g, diff(g.codes, u.codes), diff(g.scales, u.scales), diff(g.biases, u.biases), gp.e, I};
+  }
+  struct Row {
+    uint16_t *h;
+    float f;  // the row factor of x (bf16)
+  };
+  DEV Row row(const Group &gp, int i) const { return {h + (size_t)(gp.p0 + i) * I, bf ? rs[R.pair_q[gp.p0 + i] / k] : 1.0f}; }
+  DEV void put2(const Group &, const Row &r, int o, float gv, float uv) const {
+    if (o >= I) return;
+    by_act(bf, [&]<bool BF>() { r.h[o] = swiglu16<BF>(BF ? gv * r.f : gv, BF ? uv * r.f : uv); });
+  }
+};
+struct QMoeDown : VMoeDown {
+  static constexpr bool RAGGED = true;
+  AffPack d;
+  DEV size_t src(const Group &gp, int i) const { return gp.p0 + i; }
+  DEV QMoeDownRows weights(const Group &gp) const { return {d, gp.e, H}; }
+  struct Row {
+    uint16_t *o;
+    float f;  // the row factor of h (bf16)
+  };
+  DEV Row row(const Group &gp, int i) const { return {o + (size_t)R.pair_q[gp.p0 + i] * H, bf ? rs[gp.p0 + i] : 1.0f}; }
+  DEV void put(const Group &, const Row &r, int c, float v, int) const {
+    by_act(bf, [&]<bool BF>() { r.o[c] = bits16<BF>(BF ? v * r.f : v); });
+  }
+};
+// From 8 tokens an expert on (on average); the images' sums go where the gathered GEMVs keep their h.
+static bool moe_many_rows(int bits, int T, int H, int E, int I, int k) {
+  return bits % 2 == 0 && (size_t)T * k >= (size_t)8 * E && (size_t)T * (H / 256) * 16 <= (size_t)T * k * 2 * I * 2;
+}
+
+template <class F>
+struct QOf;
+template <int BITS, int GS, bool BF16S>
+struct QOf<FAffineN<BITS, GS, BF16S>> {
+  static constexpr bool EVEN = BITS % 2 == 0;
+  using type = QAffine<BITS, GS, BF16S>;
+};
+
 template <class F>
 static int moe_ffn_affine(const void *x, int T, int H, int E, int I, int k, const AffPack &gate, const AffPack &up,
                           const AffPack &down, const MoeTokens &rt, uint16_t *h, uint16_t *gu, uint16_t *o,
@@ -1019,7 +1134,6 @@ static int moe_ffn_affine(const void *x, int T, int H, int E, int I, int k, cons
   const uint16_t *h16;
   const float *rsh;
   const int amax = std::min(E, T * k);
-  const size_t total = (size_t)T * H;
   if (gathered_gemv(T, H, I, k)) {  // as moe_ffn: every (token, slot) pair a GEMV, two launches
     const int P = T * k;
     typename FMoeGateUpA<F>::Args ga{};
@@ -1037,6 +1151,27 @@ static int moe_ffn_affine(const void *x, int T, int H, int E, int I, int k, cons
     return launch_gemv<FMoeDownA<F>>(da, h16, y, st);
   }
   const int tiles_gu = 2 * ((I + 15) / 16), tiles_dn = (H + 15) / 16;
+  if constexpr (QOf<F>::EVEN)
+    if (moe_many_rows(2, T, H, E, I, k)) {  // x: as the caller gave it
+      using Q = typename QOf<F>::type;
+      const int dt = ma.bf ? ISHZ_DT_BF16 : ISHZ_DT_F16, P = T * k;
+      const int mbs = std::min((T + 63) / 64, (4 * P / E + 63) / 64);  // row blocks for four times an even share
+      float *X = (float *)gu, *rsx = (float *)((char *)ma.ximg + q256((size_t)T * H * 2)),
+            *rsh2 = (float *)((char *)ma.himg + q256((size_t)P * I * 2));
+      int rc = launch_qimage<Q>(x, dt, T, H, ma.ximg, X, rsx, st);
+      if (rc) return rc;
+      QMoeGateUp qg{};
+      static_cast<VMoeGateUp &>(qg) = VMoeGateUp{nullptr, nullptr, nullptr, 0, H, I, R, h, k, ma.bf ? rsx : nullptr, ma.bf};
+      qg.g = gate;
+      qg.u = up;
+      if ((rc = launch_qgemm<Q>(qg, T, H, tiles_gu * 16, amax, 1, ma.ximg, X, st, mbs))) return rc;
+      if ((rc = launch_qimage<Q>(h, dt, P, I, ma.himg, X, rsh2, st))) return rc;
+      QMoeDown qd{};
+      static_cast<VMoeDown &>(qd) = VMoeDown{nullptr, nullptr, 0, I, H, R, o, ma.bf ? rsh2 : nullptr, ma.bf};
+      qd.d = down;
+      if ((rc = launch_qgemm<Q>(qd, T, I, H, amax, 1, ma.himg, X, st, mbs))) return rc;
+      return moe_combine(o, H, T, k, R, shared, shared_gate, y, ma.bf, st);
+    }
   const int act = std::min(amax, 128);
   auto pick = [&](int tiles, int even) {  // two workgroups per CU (one measured slower here)
     int t = std::max(1, std::min(32, tiles * act / (gemv_num_cu() * 2)));
@@ -1055,10 +1190,7 @@ static int moe_ffn_affine(const void *x, int T, int H, int E, int I, int k, cons
   dn.d = down;
   rc = moe_vgemm<F>(dn, T, E, k, I, H, amax, pick(tiles_dn, 0), st);
   if (rc) return rc;
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)std::min<size_t>((total + 255) / 256, 4096)), dim3(256), 0,
-                     st, o, H, T, k, R, shared, shared_gate, (uint16_t *)y, ma.bf);
-  ISHZ_LAUNCH_CHECK("moe combine launch");
-  return ISHZ_OK;
+  return moe_combine(o, H, T, k, R, shared, shared_gate, y, ma.bf, st);
 }
 
 // The affine experts of the widths other than 4 and 8 bits (2, 3 and 5 to 7): instantiated in
@@ -1124,7 +1256,7 @@ extern "C" int ishz_moe_swiglu(uint32_t type, const void *x, int x_dtype, int T,
   uint16_t *h = (uint16_t *)((uint8_t *)workspace + L.h), *o = (uint16_t *)((uint8_t *)workspace + L.o);
   uint16_t *gu = (uint16_t *)((uint8_t *)workspace + L.gu);
   const uint16_t *sh = (const uint16_t *)shared, *sg = (const uint16_t *)shared_gate;
-  MoeAct ma{x_dtype == ISHZ_DT_BF16, nullptr, (uint8_t *)workspace + L.himg};
+  MoeAct ma{x_dtype == ISHZ_DT_BF16, nullptr, (uint8_t *)workspace + L.himg, (uint8_t *)workspace + L.ximg};
   if (ma.bf) {  // the model's activations in bf16 (MoEBlock runs in x.dtype): x's fp16 image
     const uint16_t *x16;
     const int rc = act_prepare(x, ISHZ_DT_BF16, T, H, (uint8_t *)workspace + L.ximg, st, &x16, &ma.rsx);
@@ -1177,8 +1309,8 @@ extern "C" int ishz_moe_swiglu_affine(const void *x, int x_dtype, int T, int H, 
   const AffPack upk{up_codes, (const uint16_t *)up_scales, (const uint16_t *)up_biases, H * bits / 32, H / group};
   const AffPack dp{down_codes, (const uint16_t *)down_scales, (const uint16_t *)down_biases, I * bits / 32, I / group};
   const bool bf = scale_dtype == ISHZ_DT_BF16;
-  MoeAct ma{x_dtype == ISHZ_DT_BF16, nullptr, (uint8_t *)workspace + L.himg};
-  if (ma.bf) {  // bf16 activations: x's fp16 image
+  MoeAct ma{x_dtype == ISHZ_DT_BF16, nullptr, (uint8_t *)workspace + L.himg, (uint8_t *)workspace + L.ximg};
+  if (ma.bf && (gathered_gemv(T, H, I, topk) || !moe_many_rows(bits, T, H, E, I, topk))) {  // bf16 activations: x's fp16 image
     const uint16_t *x16;
     const int rc = act_prepare(x, ISHZ_DT_BF16, T, H, (uint8_t *)workspace + L.ximg, st, &x16, &ma.rsx);
     if (rc) return rc;

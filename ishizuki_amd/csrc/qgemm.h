@@ -33,11 +33,13 @@
 //   NX, float bias(raw, g, i)            fp32 MFMAs per step, and the B value of lane group g in the i-th
 //   XLEN, int xpos(q)                    their x sums: sum q of the step (over XLEN values) is A entry 4 i + g
 //   void place(step, r, v)               where the image holds values 8 r .. 8 r + 7 of a step
+//   OCC                                  workgroups of 64 rows a CU is to hold (registers)
 //   MT_MAX                               8 where the decode outweighs the products (see qgemm_mt), else 4
 #pragma once
 #include <algorithm>
 
 #include "affine_fmt.h"
+#include "affine_nbit.h"
 #include "common.h"
 
 namespace ishz {
@@ -111,10 +113,11 @@ __global__ __launch_bounds__(1024) void qimage_kernel(const uint16_t *__restrict
 #define ISHZ_WAIT_BARRIER(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory")
 
 // A problem P: bool group(z, Group &); int count(g) rows of x, rows(g) weight rows; size_t src(g, i)
-// the image row of row i; F::Args weights(g); void put(g, i, row, v, part) one output (of part
-// blockIdx.x % S of K).
+// the image row of row i; F::Args weights(g); Row row(g, i), what is to be known of output row i; void
+// put(g, row, c, v, part) one output (of part blockIdx.x % S of K), or void put2(g, row, o, v0, v1), column o = n of the wave's first column tile and of its second.
 template <class F, class P, int MT, int NT>
-__global__ __launch_bounds__(256, MT == 4 ? 3 : 2) void qgemm_kernel(P p, const u4 *__restrict__ img, const float *__restrict__ X, int K, int S) {
+__global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, const u4 *__restrict__ img, const float *__restrict__ X, int K, int S) {
+  constexpr bool RAGGED = requires { P::RAGGED; };
   static_assert(F::SEGB == 0 || F::SEGB == 2 || F::SEGB == 8, "a chunk is one group, or part of a super-block");
   constexpr int QB = 2, NB = MT == 4 ? 3 : 4, CPS = 8 / QB;  // MFMAs per chunk, chunks in LDS, chunks per step
   static_assert(MT % 4 == 0, "four waves stage the row tiles");
@@ -127,153 +130,163 @@ __global__ __launch_bounds__(256, MT == 4 ? 3 : 2) void qgemm_kernel(P p, const 
   // row tiles dealt evenly to the workgroups of a column block
   const int mtiles = (count + 15) / 16, mb = (mtiles + MT - 1) / MT;
   if ((int)blockIdx.y >= mb) return;
-  const int t0 = mtiles * (int)blockIdx.y / mb, mt = mtiles * ((int)blockIdx.y + 1) / mb - t0;
   const int part = blockIdx.x % S, c0 = (blockIdx.x / S * 4 + wave) * 16 * NT;
   const int jb = part * steps / S, je = (part + 1) * steps / S;  // this part's steps of K
   u4 *abuf = qlds;                                  // [NB][MT][QB][64]
   float *xbuf = (float *)(abuf + NB * MT * QB * 64);     // [2][NX][MT][64]
   char *extra = (char *)(xbuf + 2 * F::NX * MT * 64);
-  const typename F::Args w = p.weights(gp);
+  const auto w = p.weights(gp);
   const typename F::Ctx ctx(w, extra, wave, lane, c0, N, NT);
 
-  const u4 *abase[MT / 4];
-  const float *xbase[MT / 4];
+  for (int y = blockIdx.y; y < mb; y += gridDim.y) {  // (one pass where the grid covers every row)
+    const int t0 = mtiles * y / mb, mt = mtiles * (y + 1) / mb - t0;
+    const u4 *abase[MT / 4];
+    const float *xbase[MT / 4];
 #pragma unroll
-  for (int tt = 0; tt < MT / 4; tt++) {
-    const size_t s = p.src(gp, min(16 * (t0 + wave + 4 * tt) + n, count - 1));
-    abase[tt] = img + s * (K / 8) + g;
-    xbase[tt] = X + s * steps * (F::NX * 4) + g;
-  }
-  // chunk c of every row tile (and with a step's first chunk its sums) into buffer c % NB; past the end
-  // the last one again, so that the number of loads under way is always known
-  const int cend = je * CPS - 1;
-  auto stage = [&](int c) {
-    const int cc = min(c, cend);
-    u4 *dst = abuf + ((c % NB) * MT + wave) * QB * 64;
+    for (int tt = 0; tt < MT / 4; tt++) {
+      const size_t s = p.src(gp, min(16 * (t0 + wave + 4 * tt) + n, count - 1));
+      abase[tt] = img + s * (K / 8) + g;
+      xbase[tt] = X + s * steps * (F::NX * 4) + g;
+    }
+    // chunk c of every row tile (and with a step's first chunk its sums) into buffer c % NB; past the end
+    // the last one again, so that the number of loads under way is always known
+    const int cend = je * CPS - 1;
+    auto stage = [&](int c) {
+      const int cc = min(c, cend);
+      u4 *dst = abuf + ((c % NB) * MT + wave) * QB * 64;
 #pragma unroll
-    for (int tt = 0; tt < MT / 4; tt++)
+      for (int tt = 0; tt < MT / 4; tt++)
 #pragma unroll
-      for (int b = 0; b < QB; b++) load16_to_lds(abase[tt] + (cc * QB + b) * 4, dst + (4 * tt * QB + b) * 64);
-    if (F::NX > 0 && c % CPS == 0)
+        for (int b = 0; b < QB; b++) load16_to_lds(abase[tt] + (cc * QB + b) * 4, dst + (4 * tt * QB + b) * 64);
+      if (F::NX > 0 && c % CPS == 0)
 #pragma unroll
-      for (int i = 0; i < F::NX; i++)
+        for (int i = 0; i < F::NX; i++)
 #pragma unroll
-        for (int tt = 0; tt < MT / 4; tt++)
-          load4_to_lds(xbase[tt] + (cc / CPS * F::NX + i) * 4, xbuf + ((((c / CPS) & 1) * F::NX + i) * MT + wave + 4 * tt) * 64);
-  };
+          for (int tt = 0; tt < MT / 4; tt++)
+            load4_to_lds(xbase[tt] + (cc / CPS * F::NX + i) * 4, xbuf + ((((c / CPS) & 1) * F::NX + i) * MT + wave + 4 * tt) * 64);
+    };
 
-  f4 acc[MT][NT], C[MT][NT];
+    f4 acc[MT][NT], C[MT][NT];
 #pragma unroll
-  for (int t = 0; t < MT; t++)
+    for (int t = 0; t < MT; t++)
 #pragma unroll
-    for (int c = 0; c < NT; c++) acc[t][c] = f4{0, 0, 0, 0};
-  F::template fetch<NT>(w, ctx, jb, jb);
+      for (int c = 0; c < NT; c++) acc[t][c] = f4{0, 0, 0, 0};
+    F::template fetch<NT>(w, ctx, jb, jb);
 #pragma unroll
-  for (int d = 0; d < NB - 1; d++) stage(jb * CPS + d);
-  typename F::Raw cur[NT];
-  for (int j = jb; j < je; j++) {
+    for (int d = 0; d < NB - 1; d++) stage(jb * CPS + d);
+    typename F::Raw cur[NT];
+    for (int j = jb; j < je; j++) {
 #pragma unroll
-    for (int q = 0; q < CPS; q++) {
-      // Chunk c = CPS j + q is here and the buffer of chunk c - 1 is free. Loads issued after c's own
-      // iteration c - (NB - 1): the chunks of the NB - 2 iterations since, with a step's sums among them
-      // where one began, and the weights of the step after next (issued at q = 0).
-      constexpr int D = NB - 1;
-      auto pending = [](int q) constexpr {
-        int v = 0;
-        for (int i = 1; i < NB - 1; i++) {  // iteration c - i staged chunk c - i + D
-          v += MT * QB / 4;
-          if ((q - i + D + 8 * CPS) % CPS == 0) v += F::NX * MT / 4;
-          if ((q - i + 8 * CPS) % CPS == F::WQ) v += F::WOPS * NT;
-        }
-        return v;
-      };
-      if (q == 0) ISHZ_WAIT_BARRIER(pending(0));
-      else if (q == 1) ISHZ_WAIT_BARRIER(pending(1));
-      else if (q == 2) ISHZ_WAIT_BARRIER(pending(2));
-      else ISHZ_WAIT_BARRIER(pending(3));
-      stage(j * CPS + q + D);
-      if (q == F::WQ) F::template fetch<NT>(w, ctx, min(j + 1, je - 1), j + 1);
-      if (q == 0)
-#pragma unroll
-        for (int c = 0; c < NT; c++) cur[c] = F::template raw<NT>(ctx, j, c);
-      const u4 *ab = abuf + ((j * CPS + q) % NB) * MT * QB * 64 + lane;
-      h8 AA[2][QB];
-#pragma unroll
-      for (int b = 0; b < QB; b++) AA[0][b] = as_h8(ab[b * 64]);
-      u4 B[NT][QB];
-#pragma unroll
-      for (int c = 0; c < NT; c++) F::template decode<QB>(cur[c], q, B[c], ctx, c);
-      // Tile t's operands are read a tile ahead, and its products (SEGB = 2) scaled a tile later, while the
-      // next tile's MFMAs run.
-      f4 T[2][NT];
-      float sc[NT];
-      if constexpr (F::SEGB == 2)
-#pragma unroll
-        for (int c = 0; c < NT; c++) sc[c] = F::scale(cur[c], q);
-      auto scaled = [&](int t) {
-#pragma unroll
-        for (int c = 0; c < NT; c++)
-#pragma unroll
-          for (int e = 0; e < 4; e++) acc[t][c][e] = fmaf(sc[c], T[t & 1][c][e], acc[t][c][e]);
-      };
-#pragma unroll
-      for (int t = 0; t < MT; t++) {
-        const h8 *A = AA[t & 1];
-        if (t + 1 < MT)
-#pragma unroll
-          for (int b = 0; b < QB; b++) AA[(t + 1) & 1][b] = as_h8(ab[((t + 1) * QB + b) * 64]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int b = 0; b < QB; b++)
-#pragma unroll
-          for (int c = 0; c < NT; c++) {
-            f4 &o = F::SEGB == 0 ? acc[t][c] : F::SEGB == 8 ? C[t][c] : T[t & 1][c];
-            const bool first = F::SEGB == 8 ? q == 0 && b == 0 : F::SEGB == 2 && b == 0;
-            o = mfma32(A[b], as_h8(B[c][b]), first ? f4{0, 0, 0, 0} : o);
+      for (int q = 0; q < CPS; q++) {
+        // Chunk c = CPS j + q is here and the buffer of chunk c - 1 is free. Loads issued after c's own
+        // iteration c - (NB - 1): the chunks of the NB - 2 iterations since, with a step's sums among them
+        // where one began, and the weights of the step after next (issued at q = 0).
+        constexpr int D = NB - 1;
+        auto pending = [](int q) constexpr {
+          int v = 0;
+          for (int i = 1; i < NB - 1; i++) {  // iteration c - i staged chunk c - i + D
+            v += MT * QB / 4;
+            if ((q - i + D + 8 * CPS) % CPS == 0) v += F::NX * MT / 4;
+            if ((q - i + 8 * CPS) % CPS == F::WQ) v += F::WOPS * NT;
           }
-        if (F::SEGB == 2 && t > 0) scaled(t - 1);
+          return v;
+        };
+        if (q == 0) ISHZ_WAIT_BARRIER(pending(0));
+        else if (q == 1) ISHZ_WAIT_BARRIER(pending(1));
+        else if (q == 2) ISHZ_WAIT_BARRIER(pending(2));
+        else ISHZ_WAIT_BARRIER(pending(3));
+        stage(j * CPS + q + D);
+        if (q == F::WQ) F::template fetch<NT>(w, ctx, min(j + 1, je - 1), j + 1);
+        if (q == 0)
+#pragma unroll
+          for (int c = 0; c < NT; c++) cur[c] = F::template raw<NT>(ctx, j, c);
+        const u4 *ab = abuf + ((j * CPS + q) % NB) * MT * QB * 64 + lane;
+        h8 AA[2][QB];
+#pragma unroll
+        for (int b = 0; b < QB; b++) AA[0][b] = as_h8(ab[b * 64]);
+        u4 B[NT][QB];
+#pragma unroll
+        for (int c = 0; c < NT; c++) F::template decode<QB>(cur[c], q, B[c], ctx, c);
+        float sc[NT];
+        if constexpr (F::SEGB == 2)
+#pragma unroll
+          for (int c = 0; c < NT; c++) sc[c] = F::scale(cur[c], q);
+        // tile t's operands are read a tile ahead; RAGGED: pairs of tiles past the workgroup's rows are left
+        // out (groups of any size; the branches cost a plain product 3 %)
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+          if (RAGGED && t % 2 == 0 && t >= mt) break;
+          const h8 *A = AA[t & 1];
+          if (t + 1 < MT)
+#pragma unroll
+            for (int b = 0; b < QB; b++) AA[(t + 1) & 1][b] = as_h8(ab[((t + 1) * QB + b) * 64]);
+          __builtin_amdgcn_sched_barrier(0);
+          f4 T[NT];
+#pragma unroll
+          for (int b = 0; b < QB; b++)
+#pragma unroll
+            for (int c = 0; c < NT; c++) {
+              f4 &o = F::SEGB == 0 ? acc[t][c] : F::SEGB == 8 ? C[t][c] : T[c];
+              const bool first = F::SEGB == 8 ? q == 0 && b == 0 : F::SEGB == 2 && b == 0;
+              o = mfma32(A[b], as_h8(B[c][b]), first ? f4{0, 0, 0, 0} : o);
+            }
+          if constexpr (F::SEGB == 2)
+#pragma unroll
+            for (int c = 0; c < NT; c++)
+#pragma unroll
+              for (int e = 0; e < 4; e++) acc[t][c][e] = fmaf(sc[c], T[c][e], acc[t][c][e]);
+        }
       }
-      if (F::SEGB == 2) scaled(MT - 1);
-    }
-    if constexpr (F::NX > 0) {
-      const float *xb = xbuf + (j & 1) * F::NX * MT * 64 + lane;
+      if constexpr (F::NX > 0) {
+        const float *xb = xbuf + (j & 1) * F::NX * MT * 64 + lane;
 #pragma unroll
-      for (int i = 0; i < F::NX; i++) {
-        float bv[NT];
+        for (int i = 0; i < F::NX; i++) {
+          float bv[NT];
 #pragma unroll
-        for (int c = 0; c < NT; c++) bv[c] = F::bias(cur[c], g, i);
+          for (int c = 0; c < NT; c++) bv[c] = F::bias(cur[c], g, i);
 #pragma unroll
-        for (int t = 0; t < MT; t++)
+          for (int t = 0; t < MT; t++) {
+            if (RAGGED && t % 2 == 0 && t >= mt) break;
 #pragma unroll
-          for (int c = 0; c < NT; c++)
-            acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(xb[(i * MT + t) * 64], bv[c], acc[t][c], 0, 0, 0);
+            for (int c = 0; c < NT; c++)
+              acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(xb[(i * MT + t) * 64], bv[c], acc[t][c], 0, 0, 0);
+          }
+        }
+      }
+      if constexpr (F::SEGB == 8) {
+#pragma unroll
+        for (int c = 0; c < NT; c++) {
+          const float sc = F::scale(cur[c], 0);
+#pragma unroll
+          for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[t][c][e] = fmaf(sc, C[t][c][e], acc[t][c][e]);
+        }
       }
     }
-    if constexpr (F::SEGB == 8) {
+    ISHZ_WAIT_BARRIER(0);  // nothing still on its way to LDS when the workgroup ends
+    // every output row's place and factor first (loads for the gathered problems), then the stores
+    typename P::Row at[MT][4];
 #pragma unroll
-      for (int c = 0; c < NT; c++) {
-        const float sc = F::scale(cur[c], 0);
+    for (int t = 0; t < MT; t++)
 #pragma unroll
-        for (int t = 0; t < MT; t++)
+      for (int e = 0; e < 4; e++) at[t][e] = p.row(gp, min(16 * (t0 + t) + 4 * g + e, count - 1));
 #pragma unroll
-          for (int e = 0; e < 4; e++) acc[t][c][e] = fmaf(sc, C[t][c][e], acc[t][c][e]);
-      }
-    }
-  }
-  ISHZ_WAIT_BARRIER(0);  // nothing still on its way to LDS when the workgroup ends
-  for (int t = 0; t < mt; t++)
-#pragma unroll
-    for (int c = 0; c < NT; c++) {
-      f4 v = acc[0][c];
-#pragma unroll
-      for (int u = 1; u < MT; u++)
-        if (t == u) v = acc[u][c];
+    for (int t = 0; t < MT; t++) {
+      if (t >= mt) break;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const int i = 16 * (t0 + t) + 4 * g + e, r = c0 + 16 * c + n;
-        if (i < count && r < N) p.put(gp, i, r, v[e], part);
+        if (16 * (t0 + t) + 4 * g + e >= count) continue;
+        if constexpr (requires { p.put2(gp, at[0][0], 0, 0.0f, 0.0f); }) {  // the wave's two column tiles go together
+          p.put2(gp, at[t][e], c0 / 2 + n, acc[t][0][e], acc[t][1][e]);
+        } else {
+#pragma unroll
+          for (int c = 0; c < NT; c++)
+            if (c0 + 16 * c + n < N) p.put(gp, at[t][e], c0 + 16 * c + n, acc[t][c][e], part);
+        }
       }
     }
+  }
 }
 
 // ------------------------------------------------------------------------------- the plain problem
@@ -290,9 +303,11 @@ struct QPlain {
   DEV int rows(const Group &) const { return N; }
   DEV size_t src(const Group &, int i) const { return i; }
   DEV A weights(const Group &) const { return w; }
-  DEV void put(const Group &, int i, int row, float v, int s) const {
-    if (part) part[((size_t)s * M + i) * N + row] = v;
-    else y.put((size_t)i * N + row, i, v);
+  typedef int Row;
+  DEV Row row(const Group &, int i) const { return i; }
+  DEV void put(const Group &, Row i, int c, float v, int s) const {
+    if (part) part[((size_t)s * M + i) * N + c] = v;
+    else y.put((size_t)i * N + c, i, v);
   }
 };
 
@@ -324,29 +339,31 @@ inline QLayout qgemm_layout(int M, int K, int N, int nx, int mt) {
 }
 
 template <class F>
-static int launch_qimage(const void *x, int dt, int M, int K, void *ws, const QLayout &l, hipStream_t st) {
+static int launch_qimage(const void *x, int dt, int M, int K, void *img, float *X, float *rs, hipStream_t st) {
   const int nt = std::min(1024, K / 8);
   hipLaunchKernelGGL((qimage_kernel<F>), dim3(M), dim3((nt + 63) / 64 * 64), 0, st, (const uint16_t *)x, dt == ISHZ_DT_BF16, K,
-                     (u4 *)ws, (float *)((char *)ws + l.X), (float *)((char *)ws + l.rs));
+                     (u4 *)img, X, rs);
   ISHZ_LAUNCH_CHECK("activation image launch");
   return ISHZ_OK;
 }
 
 template <class F, class P, int MT>
-static int launch_qgemm_mt(const P &p, int mmax, int K, int N, int groups, int S, const void *ws, const QLayout &l, hipStream_t st) {
+static int launch_qgemm_mt(const P &p, int mmax, int mbs, int K, int N, int groups, int S, const void *img, const float *X, hipStream_t st) {
   const size_t lds = (size_t)(MT == 4 ? 3 : 4) * MT * 2 * 64 * 16 + (size_t)2 * F::NX * MT * 64 * 4 + F::lds_bytes(QNT);
   hipLaunchKernelGGL((qgemm_kernel<F, P, MT, QNT>),
-                     dim3((N + 64 * QNT - 1) / (64 * QNT) * S, (mmax + 16 * MT - 1) / (16 * MT), groups), dim3(256), lds, st, p,
-                     (const u4 *)ws, (const float *)((const char *)ws + l.X), K, S);
+                     dim3((N + 64 * QNT - 1) / (64 * QNT) * S, mbs ? mbs : (mmax + 16 * MT - 1) / (16 * MT), groups), dim3(256), lds, st, p,
+                     (const u4 *)img, X, K, S);
   ISHZ_LAUNCH_CHECK("many-row matmul launch");
   return ISHZ_OK;
 }
-// mmax: the most rows a group has.
+// mmax: the most rows a group can have; mbs: the row blocks to launch where few groups will have that many
+// (0: all; a workgroup takes every mbs-th block).
 template <class F, class P>
-static int launch_qgemm(const P &p, int mmax, int K, int N, int groups, int S, const void *ws, const QLayout &l, hipStream_t st) {
+static int launch_qgemm(const P &p, int mmax, int K, int N, int groups, int S, const void *img, const float *X, hipStream_t st,
+                        int mbs = 0) {
   if constexpr (F::MT_MAX == 8)
-    if (qgemm_mt(8, mmax) == 8) return launch_qgemm_mt<F, P, 8>(p, mmax, K, N, groups, S, ws, l, st);
-  return launch_qgemm_mt<F, P, 4>(p, mmax, K, N, groups, S, ws, l, st);
+    if (qgemm_mt(8, mmax) == 8) return launch_qgemm_mt<F, P, 8>(p, mmax, mbs, K, N, groups, S, img, X, st);
+  return launch_qgemm_mt<F, P, 4>(p, mmax, mbs, K, N, groups, S, img, X, st);
 }
 
 // ------------------------------------------------------------------------------- MLX affine packs
@@ -366,22 +383,27 @@ DEV uint32_t pk_fma(uint32_t t, float m, float a) {  // halves t * m + a (exact 
 
 template <int BITS, int GS, bool BF16S>
 struct QAffine {
-  static constexpr int WPL = BITS / 2, SEGB = 2, NX = 1, XLEN = 64, MT_MAX = 4, WOPS = WPL + 1;
+  static constexpr int WPL = BITS / 2, SEGB = 2, NX = 1, XLEN = 64, MT_MAX = 4, OCC = BITS == 8 ? 2 : 3, WOPS = WPL + 1;
   // a wave's step of weights in LDS (read into registers with the step's first chunk, so the next step's
   // loads follow from the second one on), per column tile: 16 rows of 32 BITS bytes of codes, then the
   // rows' scales and biases of the step (8 bytes each; 4 for groups of 128)
   static constexpr int TILE = 512 * BITS + 256, WQ = 1;
   static size_t lds_bytes(int nt) { return (size_t)4 * nt * TILE; }
+  // Args: anything with AffRow arow(row)
   struct Args {
     const uint32_t *codes;
     const uint16_t *scales, *biases;
     int K;
+    DEV AffRow arow(int row) const {
+      return {codes + (size_t)row * (K * BITS / 32), scales + (size_t)row * (K / GS), biases + (size_t)row * (K / GS)};
+    }
   };
   struct Ctx {
     char *buf;
     int lane, c0, N;
     uint32_t mg;
-    DEV Ctx(const Args &, char *extra, int wave, int lane_, int c0_, int N_, int nt)
+    template <class A>
+    DEV Ctx(const A &, char *extra, int wave, int lane_, int c0_, int N_, int nt)
           : buf(extra + wave * nt * TILE), lane(lane_), c0(c0_), N(N_), mg(vconst(0x64006400u)) {}
   };
   struct Raw {
@@ -390,19 +412,20 @@ struct QAffine {
     uint32_t b;
   };
   static DEV float ld_s(uint32_t v) { return BF16S ? __builtin_bit_cast(float, v << 16) : h2f(v); }
-  template <int NT>
-  static DEV void fetch(const Args &a, const Ctx &c, int j, int) {
+  template <int NT, class A>
+  static DEV void fetch(const A &a, const Ctx &c, int j, int) {
 #pragma unroll
     for (int t = 0; t < NT; t++) {
       char *dst = c.buf + t * TILE;
 #pragma unroll
       for (int i = 0; i < WPL; i++) {
         const int q = i * 64 + c.lane, row = min(c.c0 + 16 * t + q / (2 * BITS), c.N - 1);
-        load16_to_lds(a.codes + (size_t)row * (a.K * BITS / 32) + j * 8 * BITS + (q % (2 * BITS)) * 4, dst + i * 1024);
+        load16_to_lds(a.arow(row).codes + j * 8 * BITS + (q % (2 * BITS)) * 4, dst + i * 1024);
       }
       // lanes 0..31 the scales, 32..63 the biases: dword l % 2 of row l / 2 (groups of 128: one dword)
       const int l = c.lane & 31, row = min(c.c0 + 16 * t + (l >> 1), c.N - 1);
-      const uint16_t *p = (c.lane < 32 ? a.scales : a.biases) + (size_t)row * (a.K / GS) + j * (256 / GS) + (GS == 64 ? 2 * (l & 1) : 0);
+      const AffRow ar = a.arow(row);
+      const uint16_t *p = (c.lane < 32 ? ar.scales : ar.biases) + j * (256 / GS) + (GS == 64 ? 2 * (l & 1) : 0);
       load4_to_lds(p, dst + 512 * BITS);
     }
   }

@@ -8,13 +8,14 @@ static int affine_rows(const void *x, int dt, int M, int K, const uint32_t *code
                        int N, void *y, void *ws, hipStream_t st) {
   using F = QAffine<BITS, GS, BF16S>;
   const QLayout l = qgemm_layout(M, K, N, F::NX, 4);
-  int rc = launch_qimage<F>(x, dt, M, K, ws, l, st);
+  float *X = (float *)((char *)ws + l.X), *rs = (float *)((char *)ws + l.rs);
+  int rc = launch_qimage<F>(x, dt, M, K, ws, X, rs, st);
   if (rc) return rc;
   const int S = qgemm_splits(M, K, N, 4, gemv_num_cu());
-  const Out o{y, dt, dt == ISHZ_DT_BF16 ? (const float *)((char *)ws + l.rs) : nullptr};
+  const Out o{y, dt, dt == ISHZ_DT_BF16 ? rs : nullptr};
   float *part = S > 1 ? (float *)((char *)ws + l.part) : nullptr;
   const QPlain<typename F::Args> p{{codes, (const uint16_t *)scales, (const uint16_t *)biases, K}, M, N, o, part};
-  if ((rc = launch_qgemm<F>(p, M, K, N, 1, S, ws, l, st)) || S == 1) return rc;
+  if ((rc = launch_qgemm<F>(p, M, K, N, 1, S, ws, X, st)) || S == 1) return rc;
   const size_t n = (size_t)M * N;
   hipLaunchKernelGGL(vgemm_sum_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 2048)), dim3(256), 0, st, part, S, n, N, o);
   ISHZ_LAUNCH_CHECK("many-row matmul sum launch");

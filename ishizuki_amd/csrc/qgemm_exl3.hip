@@ -13,7 +13,7 @@ template <int KA, bool HALF, int CB>
 struct QExl3 {
   using TR = Trellis<KA, HALF>;
   using T32 = Trellis32<KA, HALF>;
-  static constexpr int SEGB = 0, NX = 0, MT_MAX = 8, XLEN = 8, W = TR::WORDS, NTC = QNT, PIECES = 4 * NTC * W, PTK = NTC * W / 4;
+  static constexpr int SEGB = 0, NX = 0, MT_MAX = 8, OCC = 3, XLEN = 8, W = TR::WORDS, NTC = QNT, PIECES = 4 * NTC * W, PTK = NTC * W / 4;
   static constexpr int WOPS = (PIECES + 63) / 64 / NTC, WQ = 0;
   static size_t lds_bytes(int) { return (size_t)4 * 2 * PIECES * 16; }
   struct Args {
@@ -81,10 +81,10 @@ template <int KA, bool HALF, int CB>
 static int exl3_rows(const void *xr, int dt, int M, int K, const int16_t *trellis, int N, void *ws, const QLayout &l, float *part,
                      int S, hipStream_t st) {
   using F = QExl3<KA, HALF, CB>;
-  const int rc = launch_qimage<F>(xr, dt, M, K, ws, l, st);
+  const int rc = launch_qimage<F>(xr, dt, M, K, ws, nullptr, (float *)((char *)ws + l.rs), st);
   if (rc) return rc;
   const QPlain<typename F::Args> p{{(const uint32_t *)trellis, N / 16}, M, N, Out{nullptr, 0, nullptr}, part};
-  return launch_qgemm<F>(p, M, K, N, 1, S, ws, l, st);
+  return launch_qgemm<F>(p, M, K, N, 1, S, ws, nullptr, st);
 }
 
 // part [S][M][N] = the K parts of xr (rotated, fp16 or bf16) . W; *rs: the bf16 rows' factors.

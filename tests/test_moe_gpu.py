@@ -382,3 +382,68 @@ def test_config4_qwen_moe_bf16(T):
         Wd[e] = oracle.dequant_rows(ggml.Q4_K, d[e * db:(e + 1) * db], H, I)
     ref, bd = moe_reference_bf16(x.float().numpy(), rid, rw, Wg, Wu, Wd)
     check_bf16(y, ref, bd, f"config4 bf16 T={T}")
+
+
+def dense_affine_experts(E, H, I, bits, group, seed):
+    packs = [synth.affine_pack_bits(E * n, k, bits, group=group, seed=seed + j, scale=0.004)
+             for j, (n, k) in enumerate(((I, H), (I, H), (H, I)))]
+    dev = [tuple(torch.from_numpy(a.reshape(E, n, -1) if a.dtype != np.uint32 else a.view(np.int32).reshape(E, n, -1)).to(DEV)
+                 for a in p) for p, n in zip(packs, (I, I, H))]
+    ws = [oracle.affine_dequant(c, s.view(np.uint16), b.view(np.uint16), E * n, k, bits, group).reshape(E, n, k)
+          for (c, s, b), (n, k) in zip(packs, ((I, H), (I, H), (H, I)))]
+    return moe.AffineExperts(*dev, bits, group, E, H, I), ws
+
+
+def dense_reference(x, ids, w, gate, up, down):
+    """(ref, bound): the FFN in float64 from dense weights, and the magnitudes forming each output."""
+    x = x.astype(np.float64)
+    ref, bound = np.zeros_like(x), np.zeros_like(x)
+    for t in range(x.shape[0]):
+        for s, e in enumerate(ids[t]):
+            g = gate[e] @ x[t]
+            h = g / (1 + np.exp(-g)) * (up[e] @ x[t])
+            ref[t] += w[t, s] * (down[e] @ h)
+            bound[t] += w[t, s] * (np.abs(down[e]) @ np.abs(h))
+    return ref, bound
+
+
+@pytest.mark.parametrize("bits,group,dt,T,E,k,H,I", [
+    (4, 64, torch.float16, 70, 4, 2, 512, 256), (4, 128, torch.bfloat16, 130, 8, 4, 256, 512),
+    (2, 64, torch.float16, 40, 4, 1, 256, 256), (8, 64, torch.bfloat16, 33, 4, 4, 512, 256),
+    (6, 64, torch.float16, 300, 4, 2, 256, 256), (3, 64, torch.float16, 70, 4, 2, 256, 256)])
+@pytest.mark.parametrize("one_expert", [False, True])
+def test_swiglu_affine_many_tokens(bits, group, dt, T, E, k, H, I, one_expert):
+    """Eight tokens an expert and more: the many-row kernel (even widths), experts of one row tile and of
+    several row blocks, every token on the same experts (more row blocks than are launched), routing in
+    launches of its own past 64 tokens."""
+    ex, (gate, up, down) = dense_affine_experts(E, H, I, bits, group, seed=bits + T)
+    x = torch.from_numpy(np.random.default_rng(T).standard_normal((T, H)).astype(np.float32)).to(dt)
+    logits = np.random.default_rng(T + 1).standard_normal((T, E)).astype(np.float32)
+    if one_expert:
+        logits[:, :k] += 20
+    print(f"moe affine many tokens bits={bits} T={T} E={E} k={k} H={H} I={I} {dt} one_expert={one_expert}", flush=True)
+    y, ids, w = moe.swiglu_affine(x.to(DEV), torch.from_numpy(logits).to(DEV), ex, top_k=k, return_routing=True)
+    rid, rw = oracle.moe_route(logits, k)
+    assert np.array_equal(ids.cpu().numpy(), rid)
+    assert np.allclose(w.cpu().numpy(), rw, rtol=1e-6, atol=1e-7)
+    ref, bound = dense_reference(x.float().numpy(), rid, rw, gate, up, down)
+    y = y.float().cpu().numpy().astype(np.float64)
+    # each intermediate (gate, up, silu, h, the slot's output) rounds to the activation type: within
+    # five half ulps of the terms' magnitudes, the last one of the output
+    u = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    lim = 5 * u * bound + u * np.abs(ref) + 1e-6
+    assert np.all(np.abs(y - ref) <= lim), f"worst {np.max(np.abs(y - ref) / lim):.3g}x the bound"
+
+
+@pytest.mark.parametrize("type_,T,E,k", [(ggml.Q4_K, 33, 4, 2), (ggml.Q6_K, 40, 4, 2), (ggml.Q4_K, 80, 16, 4)])
+def test_swiglu_more_than_four_tokens_an_expert(type_, T, E, k):
+    """The sixteen-row kernel over experts: passes of sixteen tokens and remainders."""
+    H, I = 512, 256
+    (g, u, d), ex = experts(E, H, I, type_, seed=T)
+    x = synth.fp16_normal((T, H), seed=T + 7)
+    logits = np.random.default_rng(T + 9).standard_normal((T, E)).astype(np.float32)
+    y, ids, w = moe.swiglu(torch.from_numpy(x).to(DEV), torch.from_numpy(logits).to(DEV), ex, top_k=k, return_routing=True)
+    rid, rw = oracle.moe_route(logits, k)
+    assert np.array_equal(ids.cpu().numpy(), rid)
+    ref, bd = moe_reference(type_, x.astype(np.float32), rid, rw, g, u, d, E, I)
+    assert_close(y.float().cpu().numpy(), ref, bound=bd, elem=MOE_ELEM, what=f"moe T={T} E={E}")
