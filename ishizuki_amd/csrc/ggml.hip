@@ -192,13 +192,11 @@ DEV void decode8(const uint8_t *p, int e, float *v) {
 }
 #pragma clang fp contract(on)
 
-DEV uint16_t f2bf(float f) {
-  uint32_t u = __builtin_bit_cast(uint32_t, f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);  // quiet NaN
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+// Two values rounded to bf16 (nearest even, a NaN stays a quiet NaN): one v_cvt_pk_bf16_f32.
+DEV uint32_t bf16_pair(float a, float b) {
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b});
 }
-
 DEV void store8(void *out, size_t idx, int dt, const float *v) {
   if (dt == ISHZ_DT_F32) {
     f4 *o = (f4 *)((float *)out + idx);
@@ -208,7 +206,7 @@ DEV void store8(void *out, size_t idx, int dt, const float *v) {
     uint32_t h[4];
     for (int i = 0; i < 4; i++)
       h[i] = dt == ISHZ_DT_F16 ? (uint32_t)f2h(v[2 * i]) | (uint32_t)f2h(v[2 * i + 1]) << 16
-                               : (uint32_t)f2bf(v[2 * i]) | (uint32_t)f2bf(v[2 * i + 1]) << 16;
+                               : bf16_pair(v[2 * i], v[2 * i + 1]);
     *(u4 *)((uint16_t *)out + idx) = u4{h[0], h[1], h[2], h[3]};
   }
 }
@@ -222,6 +220,32 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t *__restrict_
     const int e = (int)(s % (BS / 8));
     float v[8];
     decode8<TYPE>(w + blk * TS, e, v);
+    store8(out, s * 8, dt, v);
+  }
+}
+
+// Q4_K: slice e of a block is the low or high nibbles of eight bytes of codes. The header is one 16-byte
+// load, the codes one of eight bytes, and a weight three fp32 operations (the byte decoder took three
+// times as many). Each store is a contiguous kilobyte of a wave: threads that take both nibbles of their
+// bytes write 64-byte halves of lines instead (61 us). 17408x5120 to bf16 75 -> 46 us, 5.0 TB/s, what a
+// large copy reaches; to fp32 117 -> 92.
+__global__ __launch_bounds__(256) void dequant_q4k_kernel(const uint8_t *__restrict__ w, size_t nslices, void *out, int dt) {
+#pragma clang fp contract(off)
+  for (size_t s = blockIdx.x * (size_t)blockDim.x + threadIdx.x; s < nslices; s += (size_t)gridDim.x * blockDim.x) {
+    const int e = (int)s & 31, j = e >> 2;  // sub-block
+    const uint8_t *p = w + (s >> 5) * 144;
+    const u4 h = ld16<2>(p);
+    const u2 q = ld8<2>(p + 16 + 32 * (j >> 1) + 8 * (e & 3));
+    int sc, m;
+    q4k_scale_min(h.y, h.z, h.w, j, sc, m);
+    const float dl = h2f(h.x & 0xffff) * (float)sc, ml = h2f(h.x >> 16) * (float)m;
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const uint32_t n = (q[i >> 2] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+      const float t = dl * (float)((n >> (8 * (i & 3))) & 0xff);
+      v[i] = t - ml;
+    }
     store8(out, s * 8, dt, v);
   }
 }
@@ -481,6 +505,13 @@ extern "C" int ishz_ggml_matmul_few(uint32_t type, const void *x, int x_dtype, i
 template <uint32_t TYPE, int BS, int TS>
 static int dequant_t(const void *w, size_t count, void *out, int dt, hipStream_t st) {
   const size_t slices = count / 8;
+  if constexpr (TYPE == ISHZ_GGML_Q4_K) {
+    // 32 workgroups a CU looping for 16-bit outputs (46 us; 52 without a loop), no loop for fp32 (92 us; 113)
+    const size_t cap = dt == ISHZ_DT_F32 ? (size_t)1 << 30 : (size_t)num_cu() * 32;
+    hipLaunchKernelGGL(dequant_q4k_kernel, dim3((unsigned)std::min<size_t>((slices + 255) / 256, cap)), dim3(256), 0, st, (const uint8_t *)w, slices, out, dt);
+    ISHZ_LAUNCH_CHECK("dequant launch");
+    return ISHZ_OK;
+  }
   const int blocks = (int)std::min<size_t>((slices + 255) / 256, (size_t)num_cu() * 32);
   hipLaunchKernelGGL((dequant_kernel<TYPE, BS, TS>), dim3(blocks), dim3(256), 0, st,
                      (const uint8_t *)w, slices, out, dt);
