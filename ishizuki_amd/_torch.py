@@ -12,7 +12,16 @@ def ptr(t):
 
 
 def stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current HIP stream's handle (as torch.cuda.current_stream().cuda_stream, whose Stream object
+    alone costs 2.6 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def device_f32(t, like):
+    """t as contiguous fp32 on like's device (None: None)."""
+    if t is None or (t.dtype is torch.float32 and t.device == like.device and t.is_contiguous()):
+        return t
+    return t.to(device=like.device, dtype=torch.float32).contiguous()
 
 
 def require_cuda(*ts):

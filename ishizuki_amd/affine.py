@@ -7,7 +7,7 @@ over libishizuki_hip. Kernel calls return None when declined, like the reference
 import torch
 
 from . import _lib
-from ._torch import DTYPES, ptr, require_cuda, stream
+from ._torch import DTYPES, device_f32, ptr, require_cuda, stream
 
 supported_rows = range(2, 9)   # VerifyMatmul.supportedRows (:12)
 
@@ -29,7 +29,7 @@ def hadamard_rotate(x, block, signs=None, inverse=False):
     shape = x.shape
     x2 = x.reshape(-1, shape[-1]).contiguous()
     y = torch.empty_like(x2)
-    s = None if signs is None else signs.to(device=x.device, dtype=torch.float32).contiguous()
+    s = device_f32(signs, x)
     rc = _lib.lib().ishz_hadamard(ptr(x2), DTYPES.get(x.dtype, -1), x2.shape[0], x2.shape[1], block,
                                   ptr(s), int(inverse), ptr(y), stream())
     if not _lib.check(rc, "hadamard"):
@@ -76,11 +76,11 @@ def linear(x, weight, scales, biases, signs=None, block=0, group_size=64, bits=2
     N = weight.shape[0]
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     L = _lib.lib()
-    ws_bytes = L.ishz_affine_workspace_size(M, K) if block and _prestage else 0
-    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
-    s = None
-    if block and signs is not None:
-        s = signs.to(device=x.device, dtype=torch.float32).contiguous()
+    # (one fp16 row of a 2-bit pack is rotated and staged in the GEMV)
+    in_gemv = M == 1 and bits == 2 and group_size in (64, 128) and x.dtype is torch.float16
+    ws_bytes = L.ishz_affine_workspace_size(M, K) if block and _prestage and not in_gemv else 0
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+    s = device_f32(signs, x) if block else None
     w, sc, b, sdt = _args(weight, scales, biases)
     rc = L.ishz_affine_linear(ptr(x), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, w, sc, b, sdt, N,
                               bits, group_size, ptr(y), ptr(ws), ws_bytes, stream())
@@ -97,9 +97,7 @@ def linear_rows(x, weight, scales, biases, signs=None, block=0, group_size=64, b
     L = _lib.lib()
     ws = torch.empty(L.ishz_affine_rows_workspace_size(M, K, N), dtype=torch.uint8, device=x.device)
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    s = None
-    if block and signs is not None:
-        s = signs.to(device=x.device, dtype=torch.float32).contiguous()
+    s = device_f32(signs, x) if block else None
     w, sc, b, sdt = _args(weight, scales, biases)
     rc = L.ishz_affine_linear_rows(ptr(x), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, w, sc, b, sdt, N, bits,
                                    group_size, ptr(y), ptr(ws), ws.numel(), stream())

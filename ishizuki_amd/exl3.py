@@ -79,7 +79,8 @@ def apply(x, t):
     """EXL3Kernels.apply: rotate in, matvec, rotate out; x [..., K] fp16 with up to 16 rows."""
     require_cuda(x, t.trellis)
     shape = x.shape
-    x2 = x.reshape(-1, t.input_dim).contiguous()
+    rows = x.dim() == 2 and shape[1] == t.input_dim
+    x2 = (x if rows else x.reshape(-1, t.input_dim)).contiguous()
     M = x2.shape[0]
     L = _lib.lib()
     ws = torch.empty(L.ishz_exl3_workspace_size(M, t.input_dim, t.output_dim), dtype=torch.uint8, device=x.device)
@@ -88,7 +89,7 @@ def apply(x, t):
                            ptr(t.svh), t.output_dim, t.bits2, t.codebook, ptr(y), ptr(ws), ws.numel(), stream())
     if not _lib.check(rc, "exl3_apply"):
         return None
-    return y.reshape(*shape[:-1], t.output_dim)
+    return y if rows else y.reshape(*shape[:-1], t.output_dim)
 
 
 def apply_rows(x, t):

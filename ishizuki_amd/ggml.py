@@ -43,7 +43,8 @@ def matvec(x, blocks, type_, output_dim):
     M, K = x.shape
     L = _lib.lib()
     y = torch.empty((M, output_dim), dtype=x.dtype, device=x.device)
-    wsb = L.ishz_ggml_workspace_size(type_, M, K, output_dim)
+    # (one row: the GEMV stages x itself; a bf16 row the GEMV does not take needs its image)
+    wsb = L.ishz_ggml_workspace_size(type_, M, K, output_dim) if M > 1 or (x.dtype is not torch.float16 and K % 256) else 0
     ws = torch.empty(wsb, dtype=torch.uint8, device=x.device) if wsb else None
     rc = L.ishz_ggml_matvec_ws(type_, ptr(x), DTYPES.get(x.dtype, -1), M, K, ptr(blocks),
                                blocks.numel() * blocks.element_size(), output_dim, ptr(y),
@@ -103,6 +104,8 @@ def apply(h, blocks, type_, output_dim):
     MI355X: up to 16 rows is one matvec call (the reference splits 5..16 rows into matmulFew calls
     of 8; here the matvec's MFMA path already decodes each weight once for all 16); more rows are
     16-row calls until the dense path pays, then the weight is expanded once and multiplied."""
+    if h.dim() == 2 and h.shape[0] <= 16:
+        return matvec(h, blocks, type_, output_dim)
     shape = h.shape
     x = h.reshape(-1, shape[-1])
     rows, K = x.shape

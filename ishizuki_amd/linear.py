@@ -71,6 +71,8 @@ class PackedLinear:
         if self.ggml is not None:
             return ggml.apply(x, self.ggml.bytes, self.ggml.type, self.output_dim)
         if self.exl3 is not None:
+            if x.dim() == 2 and 0 < x.shape[0] <= 16:
+                return exl3.apply(x, self.exl3)
             shape = x.shape
             rows = x.reshape(-1, shape[-1])
             y = exl3.apply_rows(rows, self.exl3) if rows.shape[0] > 16 else None
@@ -82,9 +84,12 @@ class PackedLinear:
             return torch.cat(parts, 0).reshape(*shape[:-1], self.output_dim)
         if self.is_dense:
             return x @ self.weight.t().to(x.dtype)
+        signs = self.signs if self.block > 0 else None
+        if x.dim() == 2 and 0 < x.shape[0] <= 16:
+            return affine.linear(x, self.weight, self.scales, self.biases, signs=signs, block=self.block,
+                                 group_size=self.group_size, bits=self.bits)
         shape = x.shape
         rows = x.reshape(-1, shape[-1])
-        signs = self.signs if self.block > 0 else None
         if rows.shape[0] > 16:
             y = affine.linear_rows(rows, self.weight, self.scales, self.biases, signs=signs, block=self.block,
                                    group_size=self.group_size, bits=self.bits)
