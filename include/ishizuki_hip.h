@@ -33,7 +33,8 @@ enum { ISHZ_OK = 0, ISHZ_DECLINED = 1, ISHZ_EINVAL = 2, ISHZ_EHIP = 3 };
      row's largest value lands in [0.5, 1); outputs are multiplied back, exactly, before their
      one narrowing). bf16 values convert exactly down to 2^-17 of their row's largest. The image
      lives in the call's workspace where the entry point takes one, else in a stream-ordered
-     temporary (hipMallocAsync).
+     temporary (hipMallocAsync); a single GGML or affine row is converted inside its GEMV and
+     needs neither.
    - fp32 x: fp32 precision. Every weight is decoded to its exact fp32 value and dotted with the
      fp32 x by fp32 FMAs (no image, no temporary), as the reference accumulates fp32 x in fp32.
    The MoE FFN takes fp16 or bf16 x (its intermediates are rounded to x's dtype). */

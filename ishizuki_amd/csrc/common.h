@@ -244,7 +244,7 @@ int einval(const std::string &why);
 inline hipStream_t S(ishz_stream_t s) { return (hipStream_t)s; }
 
 // bf16 activations are converted once per call into an fp16 image with a power-of-two factor per
-// row, and every kernel stages that image as it stages fp16 x:
+// row (one row: by the GEMV while it stages x), and every kernel stages that image as it stages fp16 x:
 //   xh[m][k] = fp16(x[m][k] * 2^-e_m),  2^(e_m - 1) <= max_k |x[m][k]| < 2^e_m,
 // outputs multiplied back by rs[m] = 2^e_m (exact) in fp32 before their one narrowing to x's
 // dtype. bf16 values (8 significant bits) land exactly down to 2^-17 of their row's largest
@@ -253,6 +253,9 @@ inline hipStream_t S(ishz_stream_t s) { return (hipStream_t)s; }
 size_t act_image_bytes(int M, int K);
 int act_prepare(const void *x, int dt, int M, int K, void *image, hipStream_t st, const uint16_t **xh,
                 const float **rs);
+// Whether the kernels that copy 16 bytes at a time straight into LDS may read from p (register loads take
+// any alignment; these are kept to whole 16 bytes).
+inline bool lds_loadable(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // A stream-ordered temporary (hipMallocAsync / hipFreeAsync) for calls without a workspace.
 struct StreamTemp {
   void *p = nullptr;

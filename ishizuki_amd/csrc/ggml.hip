@@ -466,7 +466,7 @@ static int ggml_call(uint32_t type, const void *x, int x_dtype, int M, int K, co
     case ISHZ_GGML_IQ2_XS: return gemv<FIQ2_XS>(xh, K, blocks, N, o, st);
     }
   }
-  if (ggml_wgemm_takes(type, M, K)) return ggml_wgemm(type, xh, M, K, blocks, N, o, ws, wb, st);
+  if (ggml_wgemm_takes(type, M, K) && lds_loadable(xh)) return ggml_wgemm(type, xh, M, K, blocks, N, o, ws, wb, st);
   switch (type) {
   case ISHZ_GGML_Q4_0: return verify<FQ4_0>(xh, M, K, blocks, N, o, st, ws, wb);
   case ISHZ_GGML_Q4_K: return verify<FQ4_K>(xh, M, K, blocks, N, o, st, ws, wb);

@@ -18,7 +18,9 @@
 //    rows are two tiles of the same workgroup, tokens are gathered through the pair list, and
 //    SwiGLU runs in the epilogue. Down works the same way and writes its rows in slot order. With
 //    up to 16 tokens every gate/up workgroup routes and places in its own LDS, so the route +
-//    place launch is skipped.
+//    place launch is skipped; past 64, routing and placement are two launches.
+//  * More than four tokens an expert (Q4_K, Q6_K): the same problems on the sixteen-row kernel
+//    (wgemm.h). From eight (affine experts of even widths): the many-row kernel (qgemm.h).
 //  * Combine: the weighted fp32 sum per token.
 // Only routed experts' blocks are ever read.
 #include <algorithm>
@@ -464,6 +466,7 @@ struct VMoeGateUp {
     g.p1 = R.offs[g.e + 1];
     return true;
   }
+  const void *xbase() const { return x; }
   DEV int count(const Group &g) const { return g.p1 - g.p0; }
   DEV int rows(const Group &) const { return 2 * ((I + 15) / 16) * 16; }
   DEV const uint16_t *xrow(const Group &g, int tk) const { return x + (size_t)(R.pair_q[g.p0 + tk] / k) * H; }
@@ -582,6 +585,7 @@ struct VMoeDown {
     g.p1 = R.offs[g.e + 1];
     return true;
   }
+  const void *xbase() const { return h; }
   DEV int count(const Group &g) const { return g.p1 - g.p0; }
   DEV int rows(const Group &) const { return H; }
   DEV const uint16_t *xrow(const Group &g, int tk) const { return h + (size_t)(g.p0 + tk) * I; }
@@ -823,7 +827,7 @@ struct WOf<FQ6_K> {
 template <class F, class P>
 static int moe_vgemm(const P &p, int T, int E, int k, int K, int rows, int groups, int tiles_per_wg, hipStream_t st) {
   if constexpr (WOf<F>::HAS && !requires { p.prologue(); })
-    if (T * k > 4 * E) return launch_wgemm<typename WOf<F>::type>(p, 16, K, rows, groups, tiles_per_wg, 1, st);
+    if (T * k > 4 * E && lds_loadable(p.xbase())) return launch_wgemm<typename WOf<F>::type>(p, 16, K, rows, groups, tiles_per_wg, 1, st);
   const int want = (2 * T * k / std::max(E, 1) + 2 + 3) / 4;
   switch (std::max(1, std::min({4, (T + 3) / 4, want}))) {
     case 1: return launch_vgemm_p<F, P, 1>(p, K, rows, groups, tiles_per_wg, st);
@@ -1113,8 +1117,10 @@ struct QMoeDown : VMoeDown {
   }
 };
 // From 8 tokens an expert on (on average); the images' sums go where the gathered GEMVs keep their h.
-static bool moe_many_rows(int bits, int T, int H, int E, int I, int k) {
-  return bits % 2 == 0 && (size_t)T * k >= (size_t)8 * E && (size_t)T * (H / 256) * 16 <= (size_t)T * k * 2 * I * 2;
+static bool moe_many_rows(int bits, int T, int H, int E, int I, int k, const AffPack &g, const AffPack &u, const AffPack &d,
+                          const void *ws) {
+  auto direct = [](const AffPack &p) { return lds_loadable(p.codes) && (uintptr_t)p.scales % 4 == 0 && (uintptr_t)p.biases % 4 == 0; };
+  return bits % 2 == 0 && direct(g) && direct(u) && direct(d) && lds_loadable(ws) && (size_t)T * k >= (size_t)8 * E && (size_t)T * (H / 256) * 16 <= (size_t)T * k * 2 * I * 2;
 }
 
 template <class F>
@@ -1152,7 +1158,7 @@ static int moe_ffn_affine(const void *x, int T, int H, int E, int I, int k, cons
   }
   const int tiles_gu = 2 * ((I + 15) / 16), tiles_dn = (H + 15) / 16;
   if constexpr (QOf<F>::EVEN)
-    if (moe_many_rows(2, T, H, E, I, k)) {  // x: as the caller gave it
+    if (moe_many_rows(2, T, H, E, I, k, gate, up, down, ma.ximg)) {  // x: as the caller gave it
       using Q = typename QOf<F>::type;
       const int dt = ma.bf ? ISHZ_DT_BF16 : ISHZ_DT_F16, P = T * k;
       const int mbs = std::min((T + 63) / 64, (4 * P / E + 63) / 64);  // row blocks for four times an even share
@@ -1310,7 +1316,7 @@ extern "C" int ishz_moe_swiglu_affine(const void *x, int x_dtype, int T, int H, 
   const AffPack dp{down_codes, (const uint16_t *)down_scales, (const uint16_t *)down_biases, I * bits / 32, I / group};
   const bool bf = scale_dtype == ISHZ_DT_BF16;
   MoeAct ma{x_dtype == ISHZ_DT_BF16, nullptr, (uint8_t *)workspace + L.himg, (uint8_t *)workspace + L.ximg};
-  if (ma.bf && (gathered_gemv(T, H, I, topk) || !moe_many_rows(bits, T, H, E, I, topk))) {  // bf16 activations: x's fp16 image
+  if (ma.bf && (gathered_gemv(T, H, I, topk) || !moe_many_rows(bits, T, H, E, I, topk, gp, upk, dp, ma.ximg))) {  // bf16 activations: x's fp16 image
     const uint16_t *x16;
     const int rc = act_prepare(x, ISHZ_DT_BF16, T, H, (uint8_t *)workspace + L.ximg, st, &x16, &ma.rsx);
     if (rc) return rc;

@@ -67,6 +67,18 @@ class PackedLinear:
         self.output_dim, self.input_dim = tensor.output_dim, tensor.input_dim
         return self
 
+    @staticmethod
+    def _many(rows, call):
+        """More than 16 rows in calls of at most 4096 (which bounds the workspace); None if there are fewer
+        or the kernel declines."""
+        n = rows.shape[0]
+        if n <= 16:
+            return None
+        if n <= 4096:
+            return call(rows)
+        parts = [call(rows[r:r + 4096]) for r in range(0, n, 4096)]
+        return None if any(p is None for p in parts) else torch.cat(parts, 0)
+
     def __call__(self, x):
         if self.ggml is not None:
             return ggml.apply(x, self.ggml.bytes, self.ggml.type, self.output_dim)
@@ -75,13 +87,13 @@ class PackedLinear:
                 return exl3.apply(x, self.exl3)
             shape = x.shape
             rows = x.reshape(-1, shape[-1])
-            y = exl3.apply_rows(rows, self.exl3) if rows.shape[0] > 16 else None
+            y = self._many(rows, lambda r: exl3.apply_rows(r, self.exl3))
             if y is not None:
                 return y.reshape(*shape[:-1], self.output_dim)
             parts = [exl3.apply(rows[r:r + 16], self.exl3) for r in range(0, rows.shape[0], 16)]
             if any(p is None for p in parts):
                 return None
-            return torch.cat(parts, 0).reshape(*shape[:-1], self.output_dim)
+            return (parts[0] if len(parts) == 1 else torch.cat(parts, 0)).reshape(*shape[:-1], self.output_dim)
         if self.is_dense:
             return x @ self.weight.t().to(x.dtype)
         signs = self.signs if self.block > 0 else None
@@ -90,13 +102,12 @@ class PackedLinear:
                                  group_size=self.group_size, bits=self.bits)
         shape = x.shape
         rows = x.reshape(-1, shape[-1])
-        if rows.shape[0] > 16:
-            y = affine.linear_rows(rows, self.weight, self.scales, self.biases, signs=signs, block=self.block,
-                                   group_size=self.group_size, bits=self.bits)
-            if y is not None:
-                return y.reshape(*shape[:-1], self.output_dim)
+        y = self._many(rows, lambda r: affine.linear_rows(r, self.weight, self.scales, self.biases, signs=signs,
+                                                          block=self.block, group_size=self.group_size, bits=self.bits))
+        if y is not None:
+            return y.reshape(*shape[:-1], self.output_dim)
         parts = [affine.linear(rows[r:r + 16], self.weight, self.scales, self.biases, signs=signs, block=self.block,
                                group_size=self.group_size, bits=self.bits) for r in range(0, rows.shape[0], 16)]
         if any(p is None for p in parts):
             return None
-        return torch.cat(parts, 0).reshape(*shape[:-1], self.output_dim)
+        return (parts[0] if len(parts) == 1 else torch.cat(parts, 0)).reshape(*shape[:-1], self.output_dim)

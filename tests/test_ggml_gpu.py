@@ -234,3 +234,15 @@ def test_sixteen_rows_per_mfma(t, M, N, K, workspace):
     assert rc == _lib.OK, _lib.last_error()
     ref, bound = ggml_reference(t, x.astype(np.float32), blk, N)
     assert_close(y.float().cpu().numpy(), ref, bound=bound, what=f"t={t} M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("M", [8, 16])
+def test_sixteen_rows_unaligned_x(M):
+    """x at an odd multiple of two bytes (a view into a larger buffer) gives the aligned call's results up to the
+    order of the sums: it takes the kernel that loads x through registers."""
+    N, K = 48, 1024
+    blk = torch.from_numpy(synth.ggml_blocks(ggml.Q4_K, N, K, seed=5, scale=1e-3)).to(DEV)
+    flat = torch.from_numpy(synth.fp16_normal((M * K + 1,), seed=6)).to(DEV)
+    x = flat[1:].view(M, K)
+    a, b = ggml.matvec(x, blk, ggml.Q4_K, N).float(), ggml.matvec(x.clone(), blk, ggml.Q4_K, N).float()
+    assert (a - b).abs().max() <= 2.0 ** -9 * b.abs().max()

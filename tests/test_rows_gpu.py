@@ -105,3 +105,32 @@ def test_exl3_rows(bits2, cb, dt, M, K, N):
     bound = np.repeat(bh.reshape(M, N // 128, 128).sum(2), 128, 1) / np.sqrt(128.0) * np.abs(svh.astype(np.float64))
     # one rounding of a rotated value to x's dtype may go the other way (fp32 butterfly order)
     check(y, ref, bound * (40 if dt == torch.bfloat16 else 5), dt, f"exl3 rows bits2={bits2} cb={cb} M={M}")
+
+
+def test_rows_decline_what_lds_loads_cannot_read():
+    """The many-row kernels read weights 16 bytes at a time straight into LDS (scales 4): other alignments are
+    declined before any launch, and PackedLinear takes the calls of 16 rows."""
+    N, K = 64, 512
+    codes, s, b = synth.affine_pack(N, K, group=64, seed=1)
+    x, _ = act(20, K, 1, torch.float16)
+    c, sd, bd = dev(codes.view(np.int32)), dev(s), dev(b)
+    off = torch.zeros(c.numel() + 1, dtype=torch.int32, device=DEV)[1:].view_as(c)
+    assert affine.linear_rows(x, off, sd, bd) is None
+    off = torch.zeros(sd.numel() + 1, dtype=torch.float16, device=DEV)[1:].view_as(sd)
+    assert affine.linear_rows(x, c, off, bd) is None and affine.linear_rows(x, c, sd, off) is None
+    tr, suh, svh = synth.exl3_pack(K, 128, bits2=4, seed=2)
+    t = exl3.EXL3Tensor(dev(tr), dev(suh), dev(svh))
+    t.trellis = torch.zeros(t.trellis.numel() + 2, dtype=torch.int16, device=DEV)[2:].view_as(t.trellis)
+    assert exl3.apply_rows(x, t) is None
+
+
+def test_packed_linear_in_blocks_of_rows():
+    """More than 4096 rows go in blocks; the rows are independent, so they equal a call of their own."""
+    from ishizuki_amd.linear import PackedLinear
+    N, K = 32, 256
+    codes, s, b = synth.affine_pack(N, K, group=64, seed=1)
+    lin = PackedLinear(dev(codes.view(np.int32)), dev(s), dev(b), group_size=64, bits=2)
+    x, _ = act(4100, K, 1, torch.float16)
+    y = lin(x)
+    assert y.shape == (4100, N)
+    assert torch.equal(y[4096:], lin(x[4000:])[96:]) and torch.equal(y[:64], lin(x[:64]))
