@@ -41,12 +41,23 @@ def _args(weight, scales, biases):
     return (ptr(weight), ptr(scales), ptr(biases), DTYPES.get(scales.dtype, -1))
 
 
+def _check_width(x, weight, scales, biases, group_size, bits):
+    """The C calls take K from x and step through the pack by it, so a pack of another width would be read
+    past its end, or in the wrong rows. (A width that is no whole number of 128 is declined there.)"""
+    N, K = weight.shape[0], x.shape[1]
+    if K % 128 == 0 and (weight.numel() * weight.element_size() * 8 != N * K * bits
+                         or scales.numel() * group_size != N * K or biases.numel() * group_size != N * K):
+        raise _lib.IshzError(f"x of width {K} through a {bits}-bit pack of {N} rows of width "
+                             f"{scales.numel() // max(N, 1) * group_size}")
+
+
 def quantized_matmul(x, weight, scales, biases, group_size=64, bits=2):
     """y = x . dequant(weight)^T for x [M, K], M in 1..16; None if declined."""
     require_cuda(x, weight, scales, biases)
     x = x.contiguous()
     M, K = x.shape
     N = weight.shape[0]
+    _check_width(x, weight, scales, biases, group_size, bits)
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     w, s, b, sdt = _args(weight, scales, biases)
     rc = _lib.lib().ishz_affine_matmul(ptr(x), DTYPES.get(x.dtype, -1), M, K, w, s, b, sdt, N, bits,
@@ -74,6 +85,7 @@ def linear(x, weight, scales, biases, signs=None, block=0, group_size=64, bits=2
     x = x.contiguous()
     M, K = x.shape
     N = weight.shape[0]
+    _check_width(x, weight, scales, biases, group_size, bits)
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     L = _lib.lib()
     # (one fp16 row of a 2-bit pack is rotated and staged in the GEMV)
@@ -94,6 +106,7 @@ def linear_rows(x, weight, scales, biases, signs=None, block=0, group_size=64, b
     x = x.contiguous()
     M, K = x.shape
     N = weight.shape[0]
+    _check_width(x, weight, scales, biases, group_size, bits)
     L = _lib.lib()
     ws = torch.empty(L.ishz_affine_rows_workspace_size(M, K, N), dtype=torch.uint8, device=x.device)
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)

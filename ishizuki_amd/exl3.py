@@ -54,10 +54,17 @@ def rotate(x, scales, before, out_dtype):
     return y
 
 
+def _check_width(x, t):
+    """The C calls take K from the tensor, so a narrower x would be read past its end."""
+    if x.dim() != 2 or x.shape[1] != t.input_dim:
+        raise _lib.IshzError(f"x of shape {tuple(x.shape)} through an EXL3 tensor of width {t.input_dim}")
+
+
 def matvec(xh, t, workspace=None):
     """xh [M, K] (already rotated; fp16, bf16 or fp32) -> fp32 [M, N]. With `workspace` (a uint8
     device tensor of matvec_workspace_size bytes) the call allocates nothing."""
     require_cuda(xh, t.trellis)
+    _check_width(xh, t)
     xh = xh.contiguous()
     M = xh.shape[0]
     y = torch.empty((M, t.output_dim), dtype=torch.float32, device=xh.device)
@@ -96,6 +103,7 @@ def apply_rows(x, t):
     """EXL3Kernels.apply for a prompt: any number of rows [M, K] in one call; None if declined (fp32 x,
     K not a multiple of 256), where `apply` takes 16 rows at a time."""
     require_cuda(x, t.trellis)
+    _check_width(x, t)
     x = x.contiguous()
     M = x.shape[0]
     L = _lib.lib()

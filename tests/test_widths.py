@@ -1,0 +1,77 @@
+"""An x whose width is not the weight's is refused before any launch (no GPU: the library is a recorder)."""
+import pytest
+import torch
+
+from ishizuki_amd import _lib, affine, exl3
+from ishizuki_amd.linear import PackedLinear
+
+
+class Recorder:
+    """Stands in for the library: every call succeeds and is listed by name."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            if name.endswith("_size"):
+                return 256
+            self.calls.append(name)
+            return _lib.OK
+        return call
+
+
+@pytest.fixture
+def library(monkeypatch):
+    lib = Recorder()
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    for m in (affine, exl3):
+        monkeypatch.setattr(m, "require_cuda", lambda *ts: None)
+        monkeypatch.setattr(m, "stream", lambda: None)
+    return lib
+
+
+def exl3_tensor(K=512, N=128):
+    return exl3.EXL3Tensor(torch.zeros(K // 16, N // 16, 32, dtype=torch.int16), torch.ones(K), torch.ones(N))
+
+
+def pack(N=8, K=512, bits=2):
+    return (torch.zeros(N, K * bits // 32, dtype=torch.int32), torch.ones(N, K // 64, dtype=torch.float16),
+            torch.zeros(N, K // 64, dtype=torch.float16))
+
+
+@pytest.mark.parametrize("rows", [3, 20, 5000])
+@pytest.mark.parametrize("width", [256, 384, 500, 640, 1024])
+def test_exl3(library, rows, width):
+    t = exl3_tensor()
+    x = torch.zeros(rows, width, dtype=torch.float16)
+    with pytest.raises(RuntimeError):
+        PackedLinear.from_exl3(t)(x)
+    with pytest.raises(RuntimeError):
+        exl3.apply_rows(x, t)
+    with pytest.raises(RuntimeError):
+        exl3.matvec(x, t)
+    if rows > 16:
+        assert library.calls == []
+
+
+@pytest.mark.parametrize("rows", [1, 3, 20, 5000])
+@pytest.mark.parametrize("width", [256, 384, 640, 1024])
+@pytest.mark.parametrize("bits", [2, 4])
+def test_affine(library, rows, width, bits):
+    p = pack(bits=bits)
+    x = torch.zeros(rows, width, dtype=torch.float16)
+    with pytest.raises(RuntimeError):
+        PackedLinear(*p, group_size=64, bits=bits)(x)
+    for f in (affine.linear_rows, affine.linear, affine.quantized_matmul):
+        with pytest.raises(RuntimeError):
+            f(x, *p, group_size=64, bits=bits)
+    assert library.calls == []
+
+
+def test_the_right_width_is_launched(library):
+    x = torch.zeros(20, 512, dtype=torch.float16)
+    assert PackedLinear.from_exl3(exl3_tensor())(x).shape == (20, 128)
+    assert PackedLinear(*pack(), group_size=64)(x).shape == (20, 8)
+    assert PackedLinear(*pack(), group_size=64)(x[:5]).shape == (5, 8)
+    assert library.calls == ["ishz_exl3_apply_rows", "ishz_affine_linear_rows", "ishz_affine_linear"]
