@@ -43,10 +43,13 @@ def _args(weight, scales, biases):
 
 def _check_width(x, weight, scales, biases, group_size, bits):
     """The C calls take K from x and step through the pack by it, so a pack of another width would be read
-    past its end, or in the wrong rows. (A width that is no whole number of 128 is declined there.)"""
+    past its end, or in the wrong rows. What they decline is left to them."""
     N, K = weight.shape[0], x.shape[1]
-    if K % 128 == 0 and (weight.numel() * weight.element_size() * 8 != N * K * bits
-                         or scales.numel() * group_size != N * K or biases.numel() * group_size != N * K):
+    if (x.dtype not in DTYPES or scales.dtype not in (torch.float16, torch.bfloat16) or not 2 <= bits <= 8
+            or group_size < 32 or group_size % 32 or K % group_size or K % 128):
+        return
+    if (weight.numel() * weight.element_size() * 8 != N * K * bits or scales.numel() * group_size != N * K
+            or biases.numel() * group_size != N * K):
         raise _lib.IshzError(f"x of width {K} through a {bits}-bit pack of {N} rows of width "
                              f"{scales.numel() // max(N, 1) * group_size}")
 

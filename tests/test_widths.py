@@ -75,3 +75,12 @@ def test_the_right_width_is_launched(library):
     assert PackedLinear(*pack(), group_size=64)(x).shape == (20, 8)
     assert PackedLinear(*pack(), group_size=64)(x[:5]).shape == (5, 8)
     assert library.calls == ["ishz_exl3_apply_rows", "ishz_affine_linear_rows", "ishz_affine_linear"]
+
+
+def test_what_the_library_declines_is_left_to_it(library):
+    """Dtypes, groups and widths it refuses reach it whatever the pack's width: the answer stays None."""
+    w, s, b = pack(K=1024)
+    x = torch.zeros(1, 512, dtype=torch.float16)
+    for kw, xx in (({"group_size": 48}, x), ({"group_size": 64}, x.to(torch.int16)), ({"group_size": 64}, x[:, :500])):
+        affine.quantized_matmul(xx, w, s, b, **kw)
+    assert library.calls == ["ishz_affine_matmul"] * 3
