@@ -112,6 +112,14 @@ __global__ __launch_bounds__(1024) void qimage_kernel(const uint16_t *__restrict
 // workgroup's barrier. (__syncthreads would wait for every load, the prefetched ones too.)
 #define ISHZ_WAIT_BARRIER(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory")
 
+// Row block y of mb takes row tiles block_tile0(n, mb, y) .. block_tile0(n, mb, y + 1) - 1 of n, dealt evenly:
+// quotient plus remainder, as n * y leaves 32 bits at about 1.5 million rows.
+__host__ __device__ constexpr int block_tile0(int n, int mb, int y) { return n / mb * y + (y < n % mb ? y : n % mb); }
+constexpr int QROWS_MAX = 65535 * 64;  // rows of one call: the row blocks of 64 a grid holds
+static_assert(block_tile0(QROWS_MAX / 16, 65535, 65535) == QROWS_MAX / 16 && block_tile0(QROWS_MAX / 16, 32768, 32767) == QROWS_MAX / 16 - 7,
+              "the last blocks of the largest call");
+static_assert(block_tile0(9, 2, 1) == 5 && block_tile0(7, 2, 1) == 4 && block_tile0(5, 5, 3) == 3, "no block over ceil(n / mb)");
+
 // A problem P: bool group(z, Group &); int count(g) rows of x, rows(g) weight rows; size_t src(g, i)
 // the image row of row i; F::Args weights(g); Row row(g, i), what is to be known of output row i; void
 // put(g, row, c, v, part) one output (of part blockIdx.x % S of K), or void put2(g, row, o, v0, v1), column o = n of the wave's first column tile and of its second.
@@ -139,7 +147,7 @@ __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, c
   const typename F::Ctx ctx(w, extra, wave, lane, c0, N, NT);
 
   for (int y = blockIdx.y; y < mb; y += gridDim.y) {  // (one pass where the grid covers every row)
-    const int t0 = mtiles * y / mb, mt = mtiles * (y + 1) / mb - t0;
+    const int t0 = block_tile0(mtiles, mb, y), mt = block_tile0(mtiles, mb, y + 1) - t0;
     const u4 *abase[MT / 4];
     const float *xbase[MT / 4];
 #pragma unroll

@@ -134,3 +134,23 @@ def test_packed_linear_in_blocks_of_rows():
     y = lin(x)
     assert y.shape == (4100, N)
     assert torch.equal(y[4096:], lin(x[4000:])[96:]) and torch.equal(y[:64], lin(x[:64]))
+
+
+@pytest.mark.parametrize("kind,M", [("affine", 1_500_017), ("exl3", 2_100_001)])
+def test_more_rows_than_a_32_bit_tile_product(kind, M):
+    """Row tile times row block passes 2^31 from 1.48 million rows (four row tiles a workgroup) and 2.1 million
+    (eight): every row equals the same row of a smaller call."""
+    K = 256
+    if kind == "affine":
+        codes, s, b = synth.affine_pack(16, K, group=64, seed=1)
+        args = (dev(codes.view(np.int32)), dev(s), dev(b))
+        call = lambda x: affine.linear_rows(x, *args)
+    else:
+        t = exl3.EXL3Tensor(*(dev(a) for a in synth.exl3_pack(K, 128, bits2=2, seed=2)))
+        call = lambda x: exl3.apply_rows(x, t)
+    print(f"rows {kind} M={M}", flush=True)
+    x = torch.randn(M, K, dtype=torch.float16, device=DEV, generator=torch.Generator(DEV).manual_seed(M))
+    y, step = call(x), 1 << 18
+    for r in range(0, M, step):
+        assert torch.equal(y[r:r + step], call(x[r:r + step])), r
+    torch.cuda.empty_cache()
