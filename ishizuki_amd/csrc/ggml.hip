@@ -376,7 +376,7 @@ __global__ __launch_bounds__(256) void vgemm_sum_kernel(const float *__restrict_
 }
 
 // Sixteen rows per MFMA (wgemm.hip).
-bool ggml_wgemm_takes(uint32_t type, int M, int K, int N);
+bool ggml_wgemm_takes(uint32_t type, int M, int K);
 size_t ggml_wgemm_part_bytes(int M, int K, int N, int cus);
 int ggml_wgemm(uint32_t type, const void *x, int M, int K, const void *w, int N, const Out &y, void *ws, size_t ws_bytes,
                hipStream_t st);
@@ -405,7 +405,7 @@ extern "C" int ishz_ggml_type_size(uint32_t type) { return type_size(type); }
 // Workspace: the activation image (bf16 / fp32 x), then the K split's fp32 parts.
 extern "C" size_t ishz_ggml_workspace_size(uint32_t type, int M, int K, int N) {
   if (!block_size(type) || M < 1 || M > 16 || K <= 0 || N <= 0) return 0;
-  if (ggml_wgemm_takes(type, M, K, N)) return act_image_bytes(M, K) + ggml_wgemm_part_bytes(M, K, N, num_cu());
+  if (ggml_wgemm_takes(type, M, K)) return act_image_bytes(M, K) + ggml_wgemm_part_bytes(M, K, N, num_cu());
   return act_image_bytes(M, K) + (K % 256 ? 0 : vgemm_workspace(M, K, N, num_cu()));
 }
 
@@ -466,7 +466,7 @@ static int ggml_call(uint32_t type, const void *x, int x_dtype, int M, int K, co
     case ISHZ_GGML_IQ2_XS: return gemv<FIQ2_XS>(xh, K, blocks, N, o, st);
     }
   }
-  if (ggml_wgemm_takes(type, M, K, N) && lds_loadable(xh)) return ggml_wgemm(type, xh, M, K, blocks, N, o, ws, wb, st);
+  if (ggml_wgemm_takes(type, M, K) && lds_loadable(xh)) return ggml_wgemm(type, xh, M, K, blocks, N, o, ws, wb, st);
   switch (type) {
   case ISHZ_GGML_Q4_0: return verify<FQ4_0>(xh, M, K, blocks, N, o, st, ws, wb);
   case ISHZ_GGML_Q4_K: return verify<FQ4_K>(xh, M, K, blocks, N, o, st, ws, wb);

@@ -9,15 +9,10 @@ namespace ishz {
 
 // From five rows on: up to four, vgemm.h's diagonal A costs one set of MFMAs too and decodes with fewer
 // instructions (17408x5120, 4 rows: Q4_K 16.6 us there, 19.7 here; Q6_K and IQ2_XS within 6 %).
-// Q4_K keeps it up to eight rows too where it splits a long K and a CU's share is large (5120x25600, 125
-// tile steps a CU, 8 rows: 26.3 us there, 26.7-27.3 here; 1024x8192, 8 steps: 13.1 and 9.0); Q6_K and
-// IQ2_XS are faster here at that shape too (46.8 and 43.1, 31.4 and 27.2).
-bool ggml_wgemm_takes(uint32_t type, int M, int K, int N) {
-  int T;
-  const int cus = gemv_num_cu();
-  if (type == ISHZ_GGML_Q4_K && M <= 8 && K % 256 == 0 && (size_t)((N + 15) / 16) * (K / 256) >= (size_t)64 * cus &&
-      vgemm_splits(M, K, N, cus, T) > 1)
-    return false;
+// Where a long K is split the two are level from five rows on (Q4_K 5120x25600, 5 to 8 rows: 24.9-25.2 us here,
+// 24.5-25.5 there; 2048x32768 18.3-18.9 and 19.4-20.6), and without a workspace, where neither splits, this one
+// is ahead (32.2-36.3 us against 41.0-43.1).
+bool ggml_wgemm_takes(uint32_t type, int M, int K) {
   return M > 4 && M <= 16 && K % 256 == 0 && (type == ISHZ_GGML_Q4_K || type == ISHZ_GGML_Q6_K || type == ISHZ_GGML_IQ2_XS);
 }
 size_t ggml_wgemm_part_bytes(int M, int K, int N, int cus) { return wgemm_part_bytes(M, K, N, cus); }
