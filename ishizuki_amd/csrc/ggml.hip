@@ -402,11 +402,13 @@ using namespace ishz;
 extern "C" int ishz_ggml_block_size(uint32_t type) { return block_size(type); }
 extern "C" int ishz_ggml_type_size(uint32_t type) { return type_size(type); }
 
-// Workspace: the activation image (bf16 / fp32 x), then the K split's fp32 parts.
+// Workspace: the activation image (bf16 x), then the K split's fp32 parts: room for either kernel's, so that a
+// workspace for 16 rows serves fewer (up to four rows are vgemm's) and x that wgemm cannot load.
 extern "C" size_t ishz_ggml_workspace_size(uint32_t type, int M, int K, int N) {
   if (!block_size(type) || M < 1 || M > 16 || K <= 0 || N <= 0) return 0;
-  if (ggml_wgemm_takes(type, M, K)) return act_image_bytes(M, K) + ggml_wgemm_part_bytes(M, K, N, num_cu());
-  return act_image_bytes(M, K) + (K % 256 ? 0 : vgemm_workspace(M, K, N, num_cu()));
+  size_t parts = K % 256 ? 0 : vgemm_workspace(M, K, N, num_cu());
+  if (ggml_wgemm_takes(type, M, K)) parts = std::max(parts, ggml_wgemm_part_bytes(M, K, N, num_cu()));
+  return act_image_bytes(M, K) + parts;
 }
 
 // x (any activation dtype) -> fp16 image; then the product with outputs in x's dtype.

@@ -246,3 +246,23 @@ def test_sixteen_rows_unaligned_x(M):
     x = flat[1:].view(M, K)
     a, b = ggml.matvec(x, blk, ggml.Q4_K, N).float(), ggml.matvec(x.clone(), blk, ggml.Q4_K, N).float()
     assert (a - b).abs().max() <= 2.0 ** -9 * b.abs().max()
+
+
+@pytest.mark.parametrize("M", [2, 4, 16])
+def test_a_larger_workspace_gives_the_same_bits(M):
+    """The workspace of 16 rows in place of the call's own: the same split, the same results (Q4_K, a K that is
+    split for two to four rows and not for sixteen)."""
+    from ishizuki_amd import _lib
+    from ishizuki_amd._torch import ptr, stream
+    L, t, N, K = _lib.lib(), ggml.Q4_K, 7000, 8192
+    blk = torch.from_numpy(synth.ggml_blocks(t, N, K, seed=1)).to(DEV)
+    x = torch.from_numpy(synth.fp16_normal((M, K), seed=M)).to(DEV)
+    ys = []
+    for rows in (M, 16):
+        wsb = L.ishz_ggml_workspace_size(t, rows, K, N)
+        ws = torch.empty(wsb, dtype=torch.uint8, device=DEV)
+        y = torch.empty((M, N), dtype=torch.float16, device=DEV)
+        rc = L.ishz_ggml_matvec_ws(t, ptr(x), 1, M, K, ptr(blk), blk.numel(), N, ptr(y), ptr(ws), wsb, stream())
+        assert rc == _lib.OK, _lib.last_error()
+        ys.append(y)
+    assert torch.equal(*ys)
