@@ -34,7 +34,7 @@ enum { ISHZ_OK = 0, ISHZ_DECLINED = 1, ISHZ_EINVAL = 2, ISHZ_EHIP = 3 };
      one narrowing). bf16 values convert exactly down to 2^-17 of their row's largest. The image
      lives in the call's workspace where the entry point takes one, else in a stream-ordered
      temporary (hipMallocAsync); a single GGML or affine row is converted inside its GEMV and
-     needs neither.
+     has no image (a rotated one still takes the workspace, for its rotation).
    - fp32 x: fp32 precision. Every weight is decoded to its exact fp32 value and dotted with the
      fp32 x by fp32 FMAs (no image, no temporary), as the reference accumulates fp32 x in fp32.
    The MoE FFN takes fp16 or bf16 x (its intermediates are rounded to x's dtype). */
@@ -139,8 +139,8 @@ int ishz_affine_matmul(const void *x, int x_dtype, int M, int K, const uint32_t 
 /* The rotated PackedLinear forward (Core/Hadamard.swift:180-231): hadamardRotate(x, block,
    signs) rounded to x's dtype, then ishz_affine_matmul. block = 0 means no rotation. For fp16
    x and M = 1 the rotation runs inside the GEMV (x is rotated while it is staged into LDS);
-   otherwise it is a separate kernel into `workspace` (ishz_affine_workspace_size bytes, which
-   bf16 / fp32 x always needs). */
+   otherwise it is a separate kernel into `workspace` (ishz_affine_workspace_size bytes).
+   Without a rotation only two and more bf16 rows need the workspace, for their fp16 image. */
 size_t ishz_affine_workspace_size(int M, int K);
 int ishz_affine_linear(const void *x, int x_dtype, int M, int K, const float *signs, int block,
                        const uint32_t *codes, const void *scales, const void *biases,

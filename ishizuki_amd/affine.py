@@ -93,7 +93,8 @@ def linear(x, weight, scales, biases, signs=None, block=0, group_size=64, bits=2
     L = _lib.lib()
     # (one fp16 row of a 2-bit pack is rotated and staged in the GEMV)
     in_gemv = M == 1 and bits == 2 and group_size in (64, 128) and x.dtype is torch.float16
-    ws_bytes = L.ishz_affine_workspace_size(M, K) if block and _prestage and not in_gemv else 0
+    image = M > 1 and x.dtype is torch.bfloat16  # two and more bf16 rows: their fp16 image
+    ws_bytes = L.ishz_affine_workspace_size(M, K) if image or (block and _prestage and not in_gemv) else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     s = device_f32(signs, x) if block else None
     w, sc, b, sdt = _args(weight, scales, biases)

@@ -647,8 +647,10 @@ extern "C" int ishz_affine_linear(const void *x, int x_dtype, int M, int K, cons
   hipStream_t st = S(stream);
   if (x_dtype != ISHZ_DT_F16) {
     // hadamardRotate in x's own dtype (Core/Hadamard.swift:8-23, the rotated activation the
-    // reference multiplies), then its fp16 image and the unrotated product
-    if (!workspace || workspace_bytes < ishz_affine_workspace_size(M, K))
+    // reference multiplies), then its fp16 image and the unrotated product. The workspace holds the
+    // rotated rows and the image of two and more
+    const bool precise = x_dtype == ISHZ_DT_F32 || (group != 64 && group != 128);
+    if ((block > 0 || (M > 1 && !precise)) && (!workspace || workspace_bytes < ishz_affine_workspace_size(M, K)))
       return einval("workspace too small (ishz_affine_workspace_size)");
     const void *xr = x;
     void *img = workspace;
@@ -657,7 +659,7 @@ extern "C" int ishz_affine_linear(const void *x, int x_dtype, int M, int K, cons
       xr = workspace;
       img = (char *)workspace + (size_t)M * K * 4;
     }
-    if (x_dtype == ISHZ_DT_F32 || (group != 64 && group != 128))
+    if (precise)
       return affine_precise(xr, x_dtype, M, K, codes, scales, biases, bf16s, N, bits, group, y, st);
     const uint16_t *xh = (const uint16_t *)xr;
     const float *rs = nullptr;

@@ -41,6 +41,26 @@ def test_affine_4bit_three_dim_input():
     assert_close(y.float().cpu().numpy(), ref, what="PackedLinear affine 4-bit")
 
 
+@pytest.mark.parametrize("bits,group", [(2, 64), (4, 64), (4, 128), (8, 64), (4, 32)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [1, 2, 4, 16, 17])
+def test_unrotated_affine_bf16_fp32(bits, group, dt, rows):
+    """A pack without a rotation and x of another type than fp16: no workspace but for the bf16 rows' image."""
+    N, K = 96, 512
+    codes, s, b = (synth.affine_pack(N, K, group=group, seed=rows) if bits == 2 else
+                   synth.affine_pack_bits(N, K, bits, group=group, seed=rows))
+    x = torch.from_numpy(synth.fp16_normal((rows, K), seed=rows + 1)).to(dt)
+    lin = PackedLinear(dev(codes.view(np.int32)), dev(s), dev(b), group_size=group, bits=bits)
+    y = lin(x.to(DEV))
+    assert y is not None and y.shape == (rows, N) and y.dtype == dt
+    xf = x.float().numpy().astype(np.float64)
+    W = oracle.affine_dequant(codes, s.view(np.uint16), b.view(np.uint16), N, K, bits, group).astype(np.float64)
+    ref = xf @ W.T
+    # fp32 sums of exact products (1e-4 of sum |x||w|, as every matmul here), then the output's rounding
+    lim = 1e-4 * (np.abs(xf) @ np.abs(W).T) + (2.0 ** -8 if dt == torch.bfloat16 else 0) * np.abs(ref)
+    assert (np.abs(y.float().cpu().numpy() - ref) <= lim).all()
+
+
 def test_ggml_blocks():
     N, K, rows = 96, 1024, 5
     blk = synth.ggml_blocks(ggml.Q6_K, N, K, seed=11)

@@ -1,4 +1,5 @@
-"""An x whose width is not the weight's is refused before any launch (no GPU: the library is a recorder)."""
+"""What the Python calls pass to the library, and what they refuse before any launch (no GPU: the library is a
+recorder)."""
 import pytest
 import torch
 
@@ -10,13 +11,14 @@ class Recorder:
     """Stands in for the library: every call succeeds and is listed by name."""
 
     def __init__(self):
-        self.calls = []
+        self.calls, self.args = [], []
 
     def __getattr__(self, name):
         def call(*args):
             if name.endswith("_size"):
                 return 256
             self.calls.append(name)
+            self.args.append(args)
             return _lib.OK
         return call
 
@@ -84,3 +86,12 @@ def test_what_the_library_declines_is_left_to_it(library):
     for kw, xx in (({"group_size": 48}, x), ({"group_size": 64}, x.to(torch.int16)), ({"group_size": 64}, x[:, :500])):
         affine.quantized_matmul(xx, w, s, b, **kw)
     assert library.calls == ["ishz_affine_matmul"] * 3
+
+
+@pytest.mark.parametrize("dt,M,block,needed", [(torch.float16, 1, 0, False), (torch.float16, 4, 0, False), (torch.bfloat16, 1, 0, False),
+                                               (torch.bfloat16, 2, 0, True), (torch.bfloat16, 16, 0, True), (torch.float32, 4, 0, False),
+                                               (torch.bfloat16, 1, 128, True), (torch.float32, 1, 128, True)])
+def test_affine_linear_workspace(library, dt, M, block, needed):
+    """The rotated rows and the image of two and more bf16 rows take a workspace; nothing else asks for one."""
+    affine.linear(torch.zeros(M, 512, dtype=dt), *pack(bits=4), signs=torch.ones(512), block=block, bits=4)
+    assert (library.args[0][-3] is not None) == needed and (library.args[0][-2] > 0) == needed
