@@ -92,11 +92,32 @@ def gather(ids, blocks, type_, input_dim, dtype=torch.bfloat16, rows=None):
     return out if _lib.check(rc, "ggml_gather") else None
 
 
-def dense_from_rows(nbytes):
-    """Fewest rows at which dequantize + fp16 GEMM beats 16-row streaming passes (measured on
-    MI355X with Q4_K, `python bench.py --policy`: 32 rows for a 2.9 MB attention projection, 48
-    for the 74 MB MLP projections)."""
-    return 32 if nbytes < 10_000_000 else 48
+# Formats whose 16-row calls are fastest beside their expansion (dense_from_rows)
+_FAST_ROWS = (Q4_K, IQ2_XS, IQ2_XXS, IQ4_XS)
+
+
+def dense_from_rows(nbytes, type_=None, output_dim=0, input_dim=0, dtype=None):
+    """Fewest rows at which dequantize + GEMM replaces 16-row streaming passes: 32 below 10 MB of blocks, else 48
+    (measured with Q4_K, `python bench.py --policy`).
+
+    With type and shape, later for large weights of four to six times as many columns as rows, where the
+    16-bit GEMM is slow whatever the rows (150 us at 5120x25600 against 30 at 17408x5120). us of the 16-row
+    calls against dequantize + GEMM, fp16:
+      5120x25600, 80 rows:  Q4_K 138 / 242, IQ2_XS 145 / 252; Q6_K 226 / 255, Q4_0 205 / 245, IQ3_S 209 / 253
+                  96 rows:  Q4_K 164 / 240, IQ2_XS 171 / 249; Q6_K 270 / 255, Q4_0 245 / 243, IQ3_S 248 / 251
+      4096x17408, 64 rows:  Q4_K  91 / 114, IQ2_XS  96 / 116; Q6_K 190 / 124, Q4_0 109 / 115, IQ3_S 109 / 116
+                  81 rows:  Q4_K 124 / 103, IQ2_XS 131 / 104
+    bf16 rows cost about 3 us a call more, which puts the second class over the line at 4096x17408 (64 rows,
+    Q4_0 124 / 115). 2560x10240 and 1024x4096 lose from 33 rows (80 rows, Q4_K: 65 / 35 and 65 / 26); IQ1_M,
+    at twice the time a call, and fp32 x, whose calls are the exact-weight kernel's, keep the first line."""
+    base = 32 if nbytes < 10_000_000 else 48
+    weights = output_dim * input_dim
+    if (weights < 64_000_000 or not 4 * output_dim <= input_dim <= 6 * output_dim or type_ == IQ1_M
+            or dtype not in (torch.float16, torch.bfloat16)):
+        return base
+    if weights < 100_000_000:
+        return 65 if type_ in _FAST_ROWS else base
+    return 96 if type_ in _FAST_ROWS else 81
 
 
 def apply(h, blocks, type_, output_dim):
@@ -111,9 +132,7 @@ def apply(h, blocks, type_, output_dim):
     rows, K = x.shape
     if rows <= 16:
         y = matvec(x, blocks, type_, output_dim)
-    # (K of four times N and more: the fp16 GEMM takes 150 us at 5120x25600 whatever the rows, so 16-row
-    # calls win longer: 80 rows Q4_K 139 us against 241, Q6_K 233 against 254, Q4_0 214 against 242)
-    elif rows < (96 if K >= 4 * output_dim else dense_from_rows(blocks.numel())):
+    elif rows < dense_from_rows(blocks.numel(), type_, output_dim, K, x.dtype):
         parts = [matvec(x[r:r + 16], blocks, type_, output_dim) for r in range(0, rows, 16)]
         y = None if any(p is None for p in parts) else torch.cat(parts, 0)
     else:

@@ -72,6 +72,19 @@ def test_ggml_blocks():
     assert_close(y.float().cpu().numpy(), ref, what="PackedLinear ggml")
 
 
+@pytest.mark.parametrize("t", [ggml.Q4_K, ggml.Q6_K, ggml.Q4_0])
+@pytest.mark.parametrize("rows,first", [(40, 96), (95, 96), (96, 96)])
+def test_ggml_prompt_on_both_sides_of_the_line(monkeypatch, t, rows, first):
+    """Up to 95 rows in 16-row calls, a remainder among them, and the expansion from 96 on: both within the
+    bound of the other."""
+    monkeypatch.setattr(ggml, "dense_from_rows", lambda *a: first)
+    N, K = 48, 512
+    blk = synth.ggml_blocks(t, N, K, seed=rows)
+    x = synth.fp16_normal((rows, K), seed=rows + 1)
+    y = PackedLinear.from_ggml(gguf.GGUFBlocks(dev(blk), t, (N, K)))(dev(x))
+    assert_close(y.float().cpu().numpy(), oracle.ggml_matmul(t, x.astype(np.float32), blk, N), what=f"ggml prompt t={t} rows={rows}")
+
+
 def test_exl3_and_dense():
     K, N, rows = 512, 256, 3
     t, suh, svh = synth.exl3_pack(K, N, bits2=4, seed=13)
