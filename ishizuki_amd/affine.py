@@ -112,10 +112,13 @@ def linear_rows(x, weight, scales, biases, signs=None, block=0, group_size=64, b
     N = weight.shape[0]
     _check_width(x, weight, scales, biases, group_size, bits)
     L = _lib.lib()
-    ws = torch.empty(L.ishz_affine_rows_workspace_size(M, K, N), dtype=torch.uint8, device=x.device)
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    # what the library declines by these is declined before anything is allocated
+    takes = x.dtype in (torch.float16, torch.bfloat16) and K % 256 == 0 and bits in (2, 4, 6, 8) and group_size in (64, 128)
+    ws_bytes = L.ishz_affine_rows_workspace_size(M, K, N) if takes else 0
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if takes else None
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device) if takes else None
     s = device_f32(signs, x) if block else None
     w, sc, b, sdt = _args(weight, scales, biases)
     rc = L.ishz_affine_linear_rows(ptr(x), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, w, sc, b, sdt, N, bits,
-                                   group_size, ptr(y), ptr(ws), ws.numel(), stream())
+                                   group_size, ptr(y), ptr(ws), ws_bytes, stream())
     return y if _lib.check(rc, "affine_linear_rows") else None

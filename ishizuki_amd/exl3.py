@@ -107,8 +107,11 @@ def apply_rows(x, t):
     x = x.contiguous()
     M = x.shape[0]
     L = _lib.lib()
-    ws = torch.empty(L.ishz_exl3_rows_workspace_size(M, t.input_dim, t.output_dim), dtype=torch.uint8, device=x.device)
-    y = torch.empty((M, t.output_dim), dtype=x.dtype, device=x.device)
+    # what the library declines by these is declined before anything is allocated
+    takes = x.dtype in (torch.float16, torch.bfloat16) and t.input_dim % 256 == 0
+    ws_bytes = L.ishz_exl3_rows_workspace_size(M, t.input_dim, t.output_dim) if takes else 0
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if takes else None
+    y = torch.empty((M, t.output_dim), dtype=x.dtype, device=x.device) if takes else None
     rc = L.ishz_exl3_apply_rows(ptr(x), DTYPES.get(x.dtype, -1), M, t.input_dim, ptr(t.trellis), ptr(t.suh), ptr(t.svh),
-                                t.output_dim, t.bits2, t.codebook, ptr(y), ptr(ws), ws.numel(), stream())
+                                t.output_dim, t.bits2, t.codebook, ptr(y), ptr(ws), ws_bytes, stream())
     return y if _lib.check(rc, "exl3_apply_rows") else None

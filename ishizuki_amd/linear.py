@@ -76,8 +76,12 @@ class PackedLinear:
             return None
         if n <= 4096:
             return call(rows)
-        parts = [call(rows[r:r + 4096]) for r in range(0, n, 4096)]
-        return None if any(p is None for p in parts) else torch.cat(parts, 0)
+        parts = []
+        for r in range(0, n, 4096):
+            parts.append(call(rows[r:r + 4096]))
+            if parts[-1] is None:
+                return None
+        return torch.cat(parts, 0)
 
     def __call__(self, x):
         if self.ggml is not None:

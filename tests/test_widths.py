@@ -8,10 +8,10 @@ from ishizuki_amd.linear import PackedLinear
 
 
 class Recorder:
-    """Stands in for the library: every call succeeds and is listed by name."""
+    """Stands in for the library: every call but the `declined` ones succeeds; all are listed."""
 
     def __init__(self):
-        self.calls, self.args = [], []
+        self.calls, self.args, self.declined = [], [], ()
 
     def __getattr__(self, name):
         def call(*args):
@@ -19,7 +19,7 @@ class Recorder:
                 return 256
             self.calls.append(name)
             self.args.append(args)
-            return _lib.OK
+            return _lib.DECLINED if name in self.declined else _lib.OK
         return call
 
 
@@ -95,3 +95,26 @@ def test_affine_linear_workspace(library, dt, M, block, needed):
     """The rotated rows and the image of two and more bf16 rows take a workspace; nothing else asks for one."""
     affine.linear(torch.zeros(M, 512, dtype=dt), *pack(bits=4), signs=torch.ones(512), block=block, bits=4)
     assert (library.args[0][-3] is not None) == needed and (library.args[0][-2] > 0) == needed
+
+
+def test_declined_prompts_allocate_nothing(library):
+    """fp32 x, odd widths, other groups and K the many-row kernels do not take: no output and no workspace is made."""
+    library.declined = ("ishz_affine_linear_rows", "ishz_exl3_apply_rows")
+    x = torch.zeros(20, 512, dtype=torch.float16)
+    grouped = tuple(t.repeat_interleave(2, 1) if t.dtype == torch.float16 else t for t in pack())  # groups of 32
+    narrow = torch.zeros(20, 384, dtype=torch.float16)
+    assert affine.linear_rows(x.float(), *pack()) is None
+    assert affine.linear_rows(x, *pack(bits=3), bits=3) is None
+    assert affine.linear_rows(x, *grouped, group_size=32) is None
+    assert affine.linear_rows(narrow, *pack(K=384)) is None
+    assert exl3.apply_rows(x.float(), exl3_tensor()) is None
+    assert exl3.apply_rows(narrow, exl3_tensor(K=384)) is None
+    for args in library.args:
+        assert args[-4:-1] == (None, None, 0)
+
+
+def test_a_declined_prompt_is_asked_once(library):
+    library.declined = ("ishz_affine_linear_rows",)
+    x = torch.zeros(9000, 512, dtype=torch.float32)
+    assert PackedLinear(*pack(), group_size=64)(x).shape == (9000, 8)
+    assert library.calls == ["ishz_affine_linear_rows"] + ["ishz_affine_linear"] * 563
