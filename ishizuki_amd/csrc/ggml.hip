@@ -510,7 +510,8 @@ static int dequant_t(const void *w, size_t count, void *out, int dt, hipStream_t
   const size_t slices = count / 8;
   if constexpr (TYPE == ISHZ_GGML_Q4_K) {
     // 32 workgroups a CU looping for 16-bit outputs (46 us; 52 without a loop), no loop for fp32 (92 us; 113)
-    const size_t cap = dt == ISHZ_DT_F32 ? (size_t)1 << 30 : (size_t)num_cu() * 32;
+    // (a launch holds less than 2^32 threads: the loop takes what is past that)
+    const size_t cap = dt == ISHZ_DT_F32 ? ((size_t)1 << 24) - 1 : (size_t)num_cu() * 32;
     hipLaunchKernelGGL(dequant_q4k_kernel, dim3((unsigned)std::min<size_t>((slices + 255) / 256, cap)), dim3(256), 0, st, (const uint8_t *)w, slices, out, dt);
     ISHZ_LAUNCH_CHECK("dequant launch");
     return ISHZ_OK;

@@ -266,3 +266,25 @@ def test_a_larger_workspace_gives_the_same_bits(M):
         assert rc == _lib.OK, _lib.last_error()
         ys.append(y)
     assert torch.equal(*ys)
+
+
+def test_dequant_more_slices_than_a_launch_has_threads():
+    """Q4_K to fp32 past 2^35 weights (2^32 slices of eight), one thread a slice below that: the first blocks, those
+    around the last thread and the last are those of small calls."""
+    nb = (1 << 27) + 5  # blocks of 256 weights
+    count = nb * 256
+    if torch.cuda.mem_get_info()[0] < count * 4 + nb * 144 + (4 << 30):
+        pytest.skip("needs 160 GB of free memory")
+    print(f"dequant {count} weights", flush=True)
+    small = torch.from_numpy(synth.ggml_blocks(ggml.Q4_K, 1, 8 * 256, seed=3)).to(DEV)
+    want = ggml.dequantize(small, ggml.Q4_K, (8 * 256,), dtype=torch.float32)
+    blk = torch.zeros(nb * 144, dtype=torch.uint8, device=DEV)
+    last = ((1 << 24) - 1) * 256 // 32  # the block after the grid's last thread
+    places = (0, last - 4, nb - 8)
+    for p in places:
+        blk[p * 144:(p + 8) * 144] = small
+    y = ggml.dequantize(blk, ggml.Q4_K, (count,), dtype=torch.float32)
+    for p in places:
+        assert torch.equal(y[p * 256:(p + 8) * 256], want), p
+    del y, blk
+    torch.cuda.empty_cache()
