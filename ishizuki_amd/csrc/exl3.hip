@@ -893,7 +893,7 @@ extern "C" int ishz_exl3_apply(const void *x, int x_dtype, int M, int K, const i
 extern "C" size_t ishz_exl3_rows_workspace_size(int M, int K, int N) {
   if (M <= 0 || K <= 0 || N <= 0 || K % 256) return 0;
   const int S = qgemm_splits(M, K, N, qgemm_mt(8, M), num_cu_e());
-  return q256((size_t)M * K * 2) + qgemm_layout(M, K, N, 0, qgemm_mt(8, M)).part + (size_t)S * M * N * 4;
+  return q256((size_t)M * K * 2) + qgemm_layout(M, K, N, false, qgemm_mt(8, M)).part + (size_t)S * M * N * 4;
 }
 
 extern "C" int ishz_exl3_apply_rows(const void *x, int x_dtype, int M, int K, const int16_t *trellis, const uint16_t *suh,
@@ -912,7 +912,7 @@ extern "C" int ishz_exl3_apply_rows(const void *x, int x_dtype, int M, int K, co
   hipStream_t st = S(stream);
   const int parts = qgemm_splits(M, K, N, qgemm_mt(8, M), num_cu_e());
   uint8_t *xr = (uint8_t *)workspace, *ws = xr + q256((size_t)M * K * 2);
-  float *yh = (float *)(ws + qgemm_layout(M, K, N, 0, qgemm_mt(8, M)).part);
+  float *yh = (float *)(ws + qgemm_layout(M, K, N, false, qgemm_mt(8, M)).part);
   if ((rc = ishz_exl3_rotate(x, x_dtype, M, K, suh, 1, xr, x_dtype, stream))) return rc;
   const float *rs;
   if ((rc = exl3_rows_core(xr, x_dtype, M, K, trellis, N, bits2, codebook, ws, yh, parts, &rs, st))) return rc;

@@ -6,8 +6,9 @@
 // up to 16 MT rows of x and 64 NT columns; a wave holds 16 NT of the columns for all of the rows, so every
 // weight is decoded by one wave of one workgroup per 16 MT rows, straight from its packed words into
 // MFMA B operands, and each 16x16x32 MFMA multiplies sixteen rows (the verify kernel's diagonal A takes
-// four). 17408x5120: 2-bit affine with the rotation, 300 rows 716 -> 106 us (19 calls of 16 rows
-// before), 4-bit affine, 512 rows 167 us (550 TFLOP/s); EXL3 2-bit, 128 rows 275 -> 60 us.
+// four). 17408x5120: 2-bit affine with the rotation, 300 rows 716 -> 99 us (19 calls of 16 rows
+// before; 105-108 over three weights in turn), 4-bit affine, 512 rows 170 us (537 TFLOP/s); EXL3 2-bit, 128
+// rows 275 -> 59 us (64-66 over three weights).
 //
 // x comes as an image (qimage_kernel): one row per token, each 256-step of it reordered into the A
 // operands of its 8 MFMAs (16 bytes per lane group g, at piece 4 b + g of the step), so a wave moves
@@ -17,10 +18,10 @@
 // wait for every load under way once a step, the prefetched chunks too (it does not count direct
 // loads), so the waits here are counted by hand.
 //
-// Scales. B holds exact small integers and the fp32 scale multiplies C: F::SEGB MFMAs share one
-// scale per column (a lane's C column is its own weight row). Terms that are a constant times a sum
-// of x (biases, mins) go through fp32 MFMAs 16x16x4 on the image's fp32 sums, so nothing is narrowed
-// on the way: the same exact products, fp32 sums, as the kernels for up to 16 rows.
+// Scales (affine packs). B holds exact small integers and the fp32 scale multiplies C: a chunk's two MFMAs
+// share one scale per column (a lane's C column is its own weight row). The biases go through one fp32 MFMA
+// 16x16x4 a step on the image's four fp32 sums of x, so nothing is narrowed on the way: the same
+// exact products, fp32 sums, as the kernels for up to 16 rows.
 //
 // A format F provides:
 //   Args, Ctx (per-wave constants), Raw (a column tile's step in registers)
@@ -28,12 +29,14 @@
 //                                        loads per tile at least, issued at chunk WQ of the step before
 //   Raw raw<NT>(ctx, j, c)               column tile c's share of lane group g, read from there
 //   void decode<QB>(raw, q, B[QB], ctx, c)   the B operands of chunk q (MFMAs QB q .. QB q + QB - 1)
-//   SEGB                                 MFMAs per scale: 8 (a super-block), 2 (a group of 64), 0: none
-//   float scale(raw, s)                  the scale of segment s of the step
-//   NX, float bias(raw, g, i)            fp32 MFMAs per step, and the B value of lane group g in the i-th
-//   XLEN, int xpos(q)                    their x sums: sum q of the step (over XLEN values) is A entry 4 i + g
+//   SCALED                               weights in groups of 64, each with a scale and a bias; else the MFMAs
+//                                        add straight into the sums
+//   float scale(raw, q), bias(raw)       the scale of chunk q, and the bias of lane group g's 64 weights
 //   void place(step, r, v)               where the image holds values 8 r .. 8 r + 7 of a step
-//   OCC                                  workgroups of 64 rows a CU is to hold (registers)
+//   OCC                                  workgroups of 64 rows a CU is to hold (registers). 6-bit packs with fp16
+//                                        scales spill three registers at three, which is ahead all the
+//                                        same: 17408x5120, 300 / 512 rows 124 / 193 us against 135 / 211 at two
+//                                        (64 rows 53 against 52; 4096x4096, 64 / 300 rows 28 / 43 against 26 / 41)
 //   MT_MAX                               8 where the decode outweighs the products (see qgemm_mt), else 4
 #pragma once
 #include <algorithm>
@@ -68,7 +71,7 @@ __global__ __launch_bounds__(1024) void qimage_kernel(const uint16_t *__restrict
   const int n8 = K / 8, nt = blockDim.x;  // K a multiple of 256: whole waves hold whole steps
   const uint8_t *src = (const uint8_t *)(x + (size_t)blockIdx.x * K);
   img += (size_t)blockIdx.x * n8;
-  X += (size_t)blockIdx.x * (K / 256) * F::NX * 4;
+  X += (size_t)blockIdx.x * (K / 256) * 4;
   u4 v[U];
   auto load = [&](int i0) {
 #pragma unroll
@@ -94,14 +97,14 @@ __global__ __launch_bounds__(1024) void qimage_kernel(const uint16_t *__restrict
       if (q >= n8) break;  // whole groups of 32 lanes leave together
       const u4 h = bf16 ? bf16_to_half8(v[u], down) : v[u];
       F::place(img + (q & ~31), q & 31, h);
-      if constexpr (F::NX > 0) {
+      if constexpr (F::SCALED) {  // the sum of each 64 values
         float s = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; e++) s = dot2(h[e], 0x3C003C00u, s);
         s += ISHZ_DPP(s, 0xB1);
-        if (F::XLEN >= 32) s += ISHZ_DPP(s, 0x4E);
-        if (F::XLEN >= 64) s += ISHZ_DPP(s, 0x141);
-        if ((q & (F::XLEN / 8 - 1)) == 0) X[(q >> 5) * F::NX * 4 + F::xpos((q & 31) / (F::XLEN / 8))] = s;
+        s += ISHZ_DPP(s, 0x4E);
+        s += ISHZ_DPP(s, 0x141);
+        if ((q & 7) == 0) X[q >> 3] = s;
       }
     }
   }
@@ -122,11 +125,11 @@ static_assert(block_tile0(9, 2, 1) == 5 && block_tile0(7, 2, 1) == 4 && block_ti
 
 // A problem P: bool group(z, Group &); int count(g) rows of x, rows(g) weight rows; size_t src(g, i)
 // the image row of row i; F::Args weights(g); Row row(g, i), what is to be known of output row i; void
-// put(g, row, c, v, part) one output (of part blockIdx.x % S of K), or void put2(g, row, o, v0, v1), column o = n of the wave's first column tile and of its second.
+// put(g, row, c, v, part) one output (of part blockIdx.x % S of K), or void put2(g, row, o, v0, v1), column o = n of
+// the wave's first column tile and of its second.
 template <class F, class P, int MT, int NT>
 __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, const u4 *__restrict__ img, const float *__restrict__ X, int K, int S) {
   constexpr bool RAGGED = requires { P::RAGGED; };
-  static_assert(F::SEGB == 0 || F::SEGB == 2 || F::SEGB == 8, "a chunk is one group, or part of a super-block");
   constexpr int QB = 2, NB = MT == 4 ? 3 : 4, CPS = 8 / QB;  // MFMAs per chunk, chunks in LDS, chunks per step
   static_assert(MT % 4 == 0, "four waves stage the row tiles");
   static_assert(F::WQ + NB - 1 < CPS, "a step's weights are requested before its first chunk of x, whose wait covers them");
@@ -141,8 +144,8 @@ __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, c
   const int part = blockIdx.x % S, c0 = (blockIdx.x / S * 4 + wave) * 16 * NT;
   const int jb = part * steps / S, je = (part + 1) * steps / S;  // this part's steps of K
   u4 *abuf = qlds;                                  // [NB][MT][QB][64]
-  float *xbuf = (float *)(abuf + NB * MT * QB * 64);     // [2][NX][MT][64]
-  char *extra = (char *)(xbuf + 2 * F::NX * MT * 64);
+  float *xbuf = (float *)(abuf + NB * MT * QB * 64);     // [2][MT][64], SCALED
+  char *extra = (char *)(xbuf + 2 * F::SCALED * MT * 64);
   const auto w = p.weights(gp);
   const typename F::Ctx ctx(w, extra, wave, lane, c0, N, NT);
 
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, c
     for (int tt = 0; tt < MT / 4; tt++) {
       const size_t s = p.src(gp, min(16 * (t0 + wave + 4 * tt) + n, count - 1));
       abase[tt] = img + s * (K / 8) + g;
-      xbase[tt] = X + s * steps * (F::NX * 4) + g;
+      xbase[tt] = X + s * steps * 4 + g;
     }
     // chunk c of every row tile (and with a step's first chunk its sums) into buffer c % NB; past the end
     // the last one again, so that the number of loads under way is always known
@@ -166,15 +169,13 @@ __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, c
       for (int tt = 0; tt < MT / 4; tt++)
 #pragma unroll
         for (int b = 0; b < QB; b++) load16_to_lds(abase[tt] + (cc * QB + b) * 4, dst + (4 * tt * QB + b) * 64);
-      if (F::NX > 0 && c % CPS == 0)
+      if (F::SCALED && c % CPS == 0)
 #pragma unroll
-        for (int i = 0; i < F::NX; i++)
-#pragma unroll
-          for (int tt = 0; tt < MT / 4; tt++)
-            load4_to_lds(xbase[tt] + (cc / CPS * F::NX + i) * 4, xbuf + ((((c / CPS) & 1) * F::NX + i) * MT + wave + 4 * tt) * 64);
+        for (int tt = 0; tt < MT / 4; tt++)
+          load4_to_lds(xbase[tt] + cc / CPS * 4, xbuf + (((c / CPS) & 1) * MT + wave + 4 * tt) * 64);
     };
 
-    f4 acc[MT][NT], C[MT][NT];
+    f4 acc[MT][NT];
 #pragma unroll
     for (int t = 0; t < MT; t++)
 #pragma unroll
@@ -194,7 +195,7 @@ __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, c
           int v = 0;
           for (int i = 1; i < NB - 1; i++) {  // iteration c - i staged chunk c - i + D
             v += MT * QB / 4;
-            if ((q - i + D + 8 * CPS) % CPS == 0) v += F::NX * MT / 4;
+            if ((q - i + D + 8 * CPS) % CPS == 0) v += F::SCALED * MT / 4;
             if ((q - i + 8 * CPS) % CPS == F::WQ) v += F::WOPS * NT;
           }
           return v;
@@ -216,7 +217,7 @@ __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, c
 #pragma unroll
         for (int c = 0; c < NT; c++) F::template decode<QB>(cur[c], q, B[c], ctx, c);
         float sc[NT];
-        if constexpr (F::SEGB == 2)
+        if constexpr (F::SCALED)
 #pragma unroll
           for (int c = 0; c < NT; c++) sc[c] = F::scale(cur[c], q);
         // tile t's operands are read a tile ahead; RAGGED: pairs of tiles past the workgroup's rows are left
@@ -234,41 +235,26 @@ __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, c
           for (int b = 0; b < QB; b++)
 #pragma unroll
             for (int c = 0; c < NT; c++) {
-              f4 &o = F::SEGB == 0 ? acc[t][c] : F::SEGB == 8 ? C[t][c] : T[c];
-              const bool first = F::SEGB == 8 ? q == 0 && b == 0 : F::SEGB == 2 && b == 0;
-              o = mfma32(A[b], as_h8(B[c][b]), first ? f4{0, 0, 0, 0} : o);
+              f4 &o = F::SCALED ? T[c] : acc[t][c];
+              o = mfma32(A[b], as_h8(B[c][b]), F::SCALED && b == 0 ? f4{0, 0, 0, 0} : o);
             }
-          if constexpr (F::SEGB == 2)
+          if constexpr (F::SCALED)
 #pragma unroll
             for (int c = 0; c < NT; c++)
 #pragma unroll
               for (int e = 0; e < 4; e++) acc[t][c][e] = fmaf(sc[c], T[c][e], acc[t][c][e]);
         }
       }
-      if constexpr (F::NX > 0) {
-        const float *xb = xbuf + (j & 1) * F::NX * MT * 64 + lane;
+      if constexpr (F::SCALED) {
+        const float *xb = xbuf + (j & 1) * MT * 64 + lane;
+        float bv[NT];
 #pragma unroll
-        for (int i = 0; i < F::NX; i++) {
-          float bv[NT];
+        for (int c = 0; c < NT; c++) bv[c] = F::bias(cur[c]);
 #pragma unroll
-          for (int c = 0; c < NT; c++) bv[c] = F::bias(cur[c], g, i);
+        for (int t = 0; t < MT; t++) {
+          if (RAGGED && t % 2 == 0 && t >= mt) break;
 #pragma unroll
-          for (int t = 0; t < MT; t++) {
-            if (RAGGED && t % 2 == 0 && t >= mt) break;
-#pragma unroll
-            for (int c = 0; c < NT; c++)
-              acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(xb[(i * MT + t) * 64], bv[c], acc[t][c], 0, 0, 0);
-          }
-        }
-      }
-      if constexpr (F::SEGB == 8) {
-#pragma unroll
-        for (int c = 0; c < NT; c++) {
-          const float sc = F::scale(cur[c], 0);
-#pragma unroll
-          for (int t = 0; t < MT; t++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[t][c][e] = fmaf(sc, C[t][c][e], acc[t][c][e]);
+          for (int c = 0; c < NT; c++) acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(xb[t * 64], bv[c], acc[t][c], 0, 0, 0);
         }
       }
     }
@@ -336,11 +322,11 @@ inline int qgemm_splits(int M, int K, int N, int mt, int cus) {
   if (blocks >= cus) return 1;
   return std::max(1, std::min({2 * cus / blocks, K / 256 / 4, 16}));
 }
-inline QLayout qgemm_layout(int M, int K, int N, int nx, int mt) {
+inline QLayout qgemm_layout(int M, int K, int N, bool scaled, int mt) {
   QLayout l;
   const int S = qgemm_splits(M, K, N, mt, gemv_num_cu());
   l.X = q256((size_t)M * K * 2);
-  l.rs = l.X + q256((size_t)M * (K / 256) * nx * 16);
+  l.rs = l.X + q256((size_t)M * (K / 256) * scaled * 16);
   l.part = l.rs + q256((size_t)M * 4);
   l.bytes = l.part + (S > 1 ? q256((size_t)S * M * N * 4) : 0);
   return l;
@@ -357,7 +343,7 @@ static int launch_qimage(const void *x, int dt, int M, int K, void *img, float *
 
 template <class F, class P, int MT>
 static int launch_qgemm_mt(const P &p, int mmax, int mbs, int K, int N, int groups, int S, const void *img, const float *X, hipStream_t st) {
-  const size_t lds = (size_t)(MT == 4 ? 3 : 4) * MT * 2 * 64 * 16 + (size_t)2 * F::NX * MT * 64 * 4 + F::lds_bytes(QNT);
+  const size_t lds = (size_t)(MT == 4 ? 3 : 4) * MT * 2 * 64 * 16 + (size_t)2 * F::SCALED * MT * 64 * 4 + F::lds_bytes(QNT);
   hipLaunchKernelGGL((qgemm_kernel<F, P, MT, QNT>),
                      dim3((N + 64 * QNT - 1) / (64 * QNT) * S, mbs ? mbs : (mmax + 16 * MT - 1) / (16 * MT), groups), dim3(256), lds, st, p,
                      (const u4 *)img, X, K, S);
@@ -391,7 +377,8 @@ DEV uint32_t pk_fma(uint32_t t, float m, float a) {  // halves t * m + a (exact 
 
 template <int BITS, int GS, bool BF16S>
 struct QAffine {
-  static constexpr int WPL = BITS / 2, SEGB = 2, NX = 1, XLEN = 64, MT_MAX = 4, OCC = BITS == 8 ? 2 : 3, WOPS = WPL + 1;
+  static constexpr bool SCALED = true;
+  static constexpr int WPL = BITS / 2, MT_MAX = 4, OCC = BITS == 8 ? 2 : 3, WOPS = WPL + 1;
   // a wave's step of weights in LDS (read into registers with the step's first chunk, so the next step's
   // loads follow from the second one on), per column tile: 16 rows of 32 BITS bytes of codes, then the
   // rows' scales and biases of the step (8 bytes each; 4 for groups of 128)
@@ -456,7 +443,7 @@ struct QAffine {
     const int i = GS == 64 ? s : s / 2;
     return ld_s((r.s[i >> 1] >> (16 * (i & 1))) & 0xffffu);
   }
-  static DEV float bias(const Raw &r, int, int) { return ld_s(r.b); }
+  static DEV float bias(const Raw &r) { return ld_s(r.b); }
   template <int QB>
   static DEV void decode(Raw &r, int q, u4 *B, const Ctx &c, int) {
     if (q == 0)
@@ -494,7 +481,6 @@ struct QAffine {
   }
   // Image: run r of eight values of the step is group r / 8, lane group (r / 2) % 4, MFMA 2 (r / 8) + r % 2;
   // 2 bits: a word's pairs are values p and p + 8, so neighbouring runs interleave.
-  static DEV int xpos(int q) { return q; }
   static DEV void place(u4 *step, int r, u4 v) {
     const int s = r & 1, dst = (2 * (r >> 3) + s) * 4 + ((r >> 1) & 3);
     if constexpr (BITS == 2) {

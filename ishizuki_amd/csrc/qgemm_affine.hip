@@ -7,7 +7,7 @@ template <int BITS, int GS, bool BF16S>
 static int affine_rows(const void *x, int dt, int M, int K, const uint32_t *codes, const void *scales, const void *biases,
                        int N, void *y, void *ws, hipStream_t st) {
   using F = QAffine<BITS, GS, BF16S>;
-  const QLayout l = qgemm_layout(M, K, N, F::NX, 4);
+  const QLayout l = qgemm_layout(M, K, N, true, 4);
   float *X = (float *)((char *)ws + l.X), *rs = (float *)((char *)ws + l.rs);
   int rc = launch_qimage<F>(x, dt, M, K, ws, X, rs, st);
   if (rc) return rc;
@@ -31,7 +31,7 @@ static size_t affine_rot_bytes(int M, int K) { return q256((size_t)M * K * 2); }
 
 extern "C" size_t ishz_affine_rows_workspace_size(int M, int K, int N) {
   if (M <= 0 || K <= 0 || N <= 0 || K % 256) return 0;
-  return affine_rot_bytes(M, K) + qgemm_layout(M, K, N, 1, 4).bytes;
+  return affine_rot_bytes(M, K) + qgemm_layout(M, K, N, true, 4).bytes;
 }
 
 extern "C" int ishz_affine_linear_rows(const void *x, int x_dtype, int M, int K, const float *signs, int block,

@@ -13,7 +13,8 @@ template <int KA, bool HALF, int CB>
 struct QExl3 {
   using TR = Trellis<KA, HALF>;
   using T32 = Trellis32<KA, HALF>;
-  static constexpr int SEGB = 0, NX = 0, MT_MAX = 8, OCC = 3, XLEN = 8, W = TR::WORDS, NTC = QNT, PIECES = 4 * NTC * W, PTK = NTC * W / 4;
+  static constexpr bool SCALED = false;
+  static constexpr int MT_MAX = 8, OCC = 3, W = TR::WORDS, NTC = QNT, PIECES = 4 * NTC * W, PTK = NTC * W / 4;
   static constexpr int WOPS = (PIECES + 63) / 64 / NTC, WQ = 0;
   static size_t lds_bytes(int) { return (size_t)4 * 2 * PIECES * 16; }
   struct Args {
@@ -46,8 +47,6 @@ struct QExl3 {
   static DEV Raw raw(const Ctx &, int j, int) {
     return {j & 1};
   }
-  static DEV float scale(const Raw &, int) { return 1.0f; }
-  static DEV float bias(const Raw &, int, int) { return 0.0f; }
   static DEV u2 decode4(const uint32_t *tile, const Ctx &c) {
     if constexpr (T32::FITS) {
       const uint32_t win = __builtin_amdgcn_alignbit(tile[c.wn.ja], tile[c.wn.jb], c.wn.amt);
@@ -68,7 +67,6 @@ struct QExl3 {
       B[b] = u4{lo.x, lo.y, hi.x, hi.y};
     }
   }
-  static DEV int xpos(int) { return 0; }
   // Run r: half r % 2 of K tile r / 2; its word i belongs to lane group i.
   static DEV void place(u4 *step, int r, u4 v) {
     uint32_t *d = (uint32_t *)(step + (r >> 2) * 4) + ((r >> 1) & 1) * 2 + (r & 1);
@@ -90,7 +88,7 @@ static int exl3_rows(const void *xr, int dt, int M, int K, const int16_t *trelli
 // part [S][M][N] = the K parts of xr (rotated, fp16 or bf16) . W; *rs: the bf16 rows' factors.
 int exl3_rows_core(const void *xr, int dt, int M, int K, const int16_t *trellis, int N, int bits2, int cb, void *ws, float *part,
                    int S, const float **rs, hipStream_t st) {
-  const QLayout l = qgemm_layout(M, K, N, 0, qgemm_mt(8, M));
+  const QLayout l = qgemm_layout(M, K, N, false, qgemm_mt(8, M));
   *rs = dt == ISHZ_DT_BF16 ? (const float *)((char *)ws + l.rs) : nullptr;
 #define ISHZ_E3(KA)                                                                                     \
   switch (cb) {                                                                                          \
