@@ -1,5 +1,5 @@
 """PackedLinear forward on the GPU, every kind of weight, against the CPU oracle (max |y - ref| <=
-1e-3 * max |ref|); more than 16 rows go through in 16-row calls."""
+1e-3 * max |ref|); more than 16 rows take the many-row kernels, or 16-row calls where those decline."""
 import numpy as np
 import pytest
 import torch
@@ -98,3 +98,19 @@ def test_exl3_and_dense():
     yd = PackedLinear.dense(dev(w))(dev(x))
     refd = x.astype(np.float32) @ w.astype(np.float32).T
     assert_close(yd.float().cpu().numpy(), refd, what="PackedLinear dense")
+
+
+@pytest.mark.parametrize("K", [512, 384])
+@pytest.mark.parametrize("shape", [(17,), (40,), (2, 65)])
+def test_exl3_prompt(K, shape):
+    """More than 16 rows of an EXL3 projection: the many-row kernel, and 16-row calls for a K it declines."""
+    N = 256
+    t, suh, svh = synth.exl3_pack(K, N, bits2=4, seed=K)
+    ten = exl3.EXL3Tensor(dev(t), dev(suh), dev(svh))
+    x = synth.fp16_normal((*shape, K), seed=16)
+    rows = x.reshape(-1, K)
+    assert (exl3.apply_rows(dev(rows), ten) is None) == (K == 384)
+    ref = np.concatenate([oracle.exl3_apply(rows[r:r + 16].astype(np.float32), t, suh, svh, 4, 0) for r in range(0, len(rows), 16)])
+    y = PackedLinear.from_exl3(ten)(dev(x))
+    assert y is not None and y.shape == (*shape, N)
+    assert_close(y.float().cpu().numpy().reshape(-1, N), ref, what=f"PackedLinear exl3 prompt K={K} {shape}")

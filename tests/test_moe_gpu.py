@@ -299,10 +299,12 @@ def check_bf16(y, ref, bound, what):
     assert not bad.any(), f"{what}: {int(bad.sum())} outside; worst {np.max(np.abs(y - ref) / lim):.3g}x"
 
 
-@pytest.mark.parametrize("T,type_", [(1, ggml.Q4_K), (2, ggml.Q6_K), (5, ggml.Q4_K), (20, ggml.Q4_0), (3, ggml.Q6_K)])
+@pytest.mark.parametrize("T,type_", [(1, ggml.Q4_K), (2, ggml.Q6_K), (5, ggml.Q4_K), (20, ggml.Q4_0), (3, ggml.Q6_K),
+                                     (18, ggml.Q4_K), (40, ggml.Q6_K)])
 def test_swiglu_bf16(T, type_):
     """The MoE FFN in bf16 (MoEBlock runs in the model's dtype): every stage's bf16 roundings,
-    bf16 x and h staged from fp16 images with a factor per row, against a bf16 restatement."""
+    bf16 x and h staged from fp16 images with a factor per row, against a bf16 restatement. More than
+    four tokens an expert (the last two): the sixteen-row kernel."""
     E, H, I, k = 16, 512, 256, 4
     (g, u, d), ex = experts(E, H, I, type_, seed=T + 100, scale=0.002)
     x = torch.from_numpy(synth.fp16_normal((T, H), seed=T + 101).astype(np.float32) * 30.0).to(torch.bfloat16)
@@ -410,12 +412,14 @@ def dense_reference(x, ids, w, gate, up, down):
 @pytest.mark.parametrize("bits,group,dt,T,E,k,H,I", [
     (4, 64, torch.float16, 70, 4, 2, 512, 256), (4, 128, torch.bfloat16, 130, 8, 4, 256, 512),
     (2, 64, torch.float16, 40, 4, 1, 256, 256), (8, 64, torch.bfloat16, 33, 4, 4, 512, 256),
-    (6, 64, torch.float16, 300, 4, 2, 256, 256), (3, 64, torch.float16, 70, 4, 2, 256, 256)])
+    (6, 64, torch.float16, 300, 4, 2, 256, 256), (3, 64, torch.float16, 70, 4, 2, 256, 256),
+    (4, 64, torch.float16, 300, 32, 2, 256, 256), (4, 64, torch.bfloat16, 300, 32, 2, 512, 256),
+    (8, 128, torch.float16, 260, 64, 3, 256, 512)])
 @pytest.mark.parametrize("one_expert", [False, True])
 def test_swiglu_affine_many_tokens(bits, group, dt, T, E, k, H, I, one_expert):
     """Eight tokens an expert and more: the many-row kernel (even widths), experts of one row tile and of
-    several row blocks, every token on the same experts (more row blocks than are launched), routing in
-    launches of its own past 64 tokens."""
+    several row blocks, every token on the same experts, routing in launches of its own past 64 tokens. The last
+    three launch one or two row blocks and need five on those experts, so a workgroup takes several in turn."""
     ex, (gate, up, down) = dense_affine_experts(E, H, I, bits, group, seed=bits + T)
     x = torch.from_numpy(np.random.default_rng(T).standard_normal((T, H)).astype(np.float32)).to(dt)
     logits = np.random.default_rng(T + 1).standard_normal((T, E)).astype(np.float32)

@@ -89,7 +89,10 @@ def test_affine_rows_declines():
     (4, 1, torch.bfloat16, 64, 1280, 128), (4, 2, torch.float16, 31, 2048, 128), (5, 2, torch.float16, 20, 256, 256),
     (6, 0, torch.float16, 33, 512, 128), (7, 2, torch.bfloat16, 20, 512, 128), (8, 1, torch.float16, 300, 768, 128),
     (10, 0, torch.float16, 17, 512, 128), (12, 2, torch.float16, 17, 512, 128), (14, 1, torch.float16, 17, 512, 128),
-    (16, 0, torch.bfloat16, 130, 512, 256)])
+    (16, 0, torch.bfloat16, 130, 512, 256),
+    # eight row tiles a workgroup and K in parts of uneven length (2 of 11 steps, 5 of 21)
+    (4, 0, torch.float16, 129, 2816, 256), (8, 2, torch.bfloat16, 129, 2816, 128), (4, 1, torch.float16, 70, 5376, 256),
+    (4, 2, torch.bfloat16, 70, 5376, 256)])
 def test_exl3_rows(bits2, cb, dt, M, K, N):
     print(f"exl3 rows bits2={bits2} cb={cb} M={M} K={K} N={N} {dt}", flush=True)
     tr, suh, svh = synth.exl3_pack(K, N, bits2=bits2, seed=bits2 + M)
