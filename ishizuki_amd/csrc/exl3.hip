@@ -137,14 +137,10 @@ __global__ __launch_bounds__(256) void exl3_mm_f32(const float *__restrict__ x, 
 }
 
 // ------------------------------------------------------------------- streaming matvec / verify
-// For rates whose four lane states span at most 32 bits: a lane's window is one v_alignbit of
+// For rates whose four lane states span at most 32 bits (Trellis32): a lane's window is one v_alignbit of
 // two tile words, each state one bit-field extract, and two weights are decoded per packed fp16
 // operation. A workgroup owns TN column tiles and its waves split the K tiles (tk = wave, wave +
 // KS, ...), keeping D steps of tile words and x in flight; partials meet in LDS at the end.
-// ------------------------------------------------------------------- streaming matvec / verify
-// For rates whose four lane states span at most 32 bits (Trellis32). A workgroup owns TN column tiles and
-// its waves split the K tiles (tk = wave, wave + KS, ...), keeping D steps of tile words and x in
-// flight; partials meet in LDS at the end.
 template <int KA, bool HALF, int CB, bool MF, int TN, int D>
 __global__ __launch_bounds__(1024) void exl3_mm2(const uint16_t *__restrict__ xh, int M, int K,
                                                 const uint32_t *__restrict__ trellis, int N,

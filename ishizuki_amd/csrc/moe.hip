@@ -807,8 +807,6 @@ struct FMoeDown : F {
   }
 };
 
-// Quads per pass sized for about twice an expert's expected load (T k / E tokens) plus two;
-// an expert with more tokens takes further passes.
 // More than four tokens an expert on average: sixteen rows per MFMA (wgemm.h) for the formats it takes.
 template <class F>
 struct WOf {
@@ -824,6 +822,8 @@ struct WOf<FQ6_K> {
   static constexpr bool HAS = true;
   using type = WQ6_K;
 };
+// Else quads per pass sized for about twice an expert's expected load (T k / E tokens) plus two;
+// an expert with more tokens takes further passes.
 template <class F, class P>
 static int moe_vgemm(const P &p, int T, int E, int k, int K, int rows, int groups, int tiles_per_wg, hipStream_t st) {
   if constexpr (WOf<F>::HAS && !requires { p.prologue(); })
