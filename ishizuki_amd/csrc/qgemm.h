@@ -259,12 +259,15 @@ __global__ __launch_bounds__(256, MT == 4 ? F::OCC : 2) void qgemm_kernel(P p, c
       }
     }
     ISHZ_WAIT_BARRIER(0);  // nothing still on its way to LDS when the workgroup ends
-    // every output row's place and factor first (loads for the gathered problems), then the stores
+    // every output row's place and factor first (loads for the gathered problems), then the stores. The loads end
+    // here: to the compiler one of them could be under way still in the next pass, and it put a wait for every
+    // load, the prefetched chunks too, into each step of K (MoE down, by chance of the registers).
     typename P::Row at[MT][4];
 #pragma unroll
     for (int t = 0; t < MT; t++)
 #pragma unroll
       for (int e = 0; e < 4; e++) at[t][e] = p.row(gp, min(16 * (t0 + t) + 4 * g + e, count - 1));
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
 #pragma unroll
     for (int t = 0; t < MT; t++) {
       if (t >= mt) break;
