@@ -98,7 +98,8 @@ _FAST_ROWS = (Q4_K, IQ2_XS, IQ2_XXS, IQ4_XS)
 
 def dense_from_rows(nbytes, type_=None, output_dim=0, input_dim=0, dtype=None):
     """Fewest rows at which dequantize + GEMM replaces 16-row streaming passes: 32 below 10 MB of blocks, else 48
-    (measured with Q4_K, `python bench.py --policy`).
+    (measured with Q4_K, whose calls are faster since: 1024x5120, 32 rows 29 us against 27; 17408x5120, 48 rows
+    64 against 75 and 64 rows 84 against 77; Q6_K and Q4_0 there lose from 32 on, 77 / 78 and 93 / 73).
 
     With type and shape, later for large weights of four to six times as many columns as rows, where the
     16-bit GEMM is slow whatever the rows (150 us at 5120x25600 against 30 at 17408x5120). us of the 16-row
