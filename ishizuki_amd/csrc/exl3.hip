@@ -903,6 +903,7 @@ extern "C" int ishz_exl3_apply_rows(const void *x, int x_dtype, int M, int K, co
   if (!x || !trellis || !suh || !svh || !y) return einval("null pointer");
   if (!lds_loadable(trellis) || !lds_loadable(workspace)) return decline("many rows: trellis and workspace aligned to 16 bytes");
   if (M > QROWS_MAX) return decline("many rows: more row blocks than a grid holds");
+  if (!one_rotation(M, std::max(K, N))) return decline("many rows: more to rotate than a launch holds");
   if (!workspace || workspace_bytes < ishz_exl3_rows_workspace_size(M, K, N))
     return einval("workspace too small (ishz_exl3_rows_workspace_size)");
   hipStream_t st = S(stream);

@@ -122,6 +122,12 @@ constexpr int QROWS_MAX = 65535 * 64;  // rows of one call: the row blocks of 64
 static_assert(block_tile0(QROWS_MAX / 16, 65535, 65535) == QROWS_MAX / 16 && block_tile0(QROWS_MAX / 16, 32768, 32767) == QROWS_MAX / 16 - 7,
               "the last blocks of the largest call");
 static_assert(block_tile0(9, 2, 1) == 5 && block_tile0(7, 2, 1) == 4 && block_tile0(5, 5, 3) == 3, "no block over ceil(n / mb)");
+// Whether the rotation of M rows of K values, 512 to a workgroup (or one larger Hadamard block), is one launch:
+// less than 2^32 threads, workgroups of 256. The rotations have no loop over workgroups.
+constexpr bool one_rotation(int M, int K, int block = 128) {
+  const size_t per = block > 128 ? block : 512;
+  return ((size_t)M * K + per - 1) / per < (size_t)1 << 24;
+}
 
 // A problem P: bool group(z, Group &); int count(g) rows of x, rows(g) weight rows; size_t src(g, i)
 // the image row of row i; F::Args weights(g); Row row(g, i), what is to be known of output row i; void

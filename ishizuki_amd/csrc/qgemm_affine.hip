@@ -48,6 +48,7 @@ extern "C" int ishz_affine_linear_rows(const void *x, int x_dtype, int M, int K,
   if (!lds_loadable(codes) || !lds_loadable(workspace) || (uintptr_t)scales % 4 || (uintptr_t)biases % 4)
     return decline("many rows: codes and workspace aligned to 16 bytes, scales and biases to 4");
   if (M > QROWS_MAX) return decline("many rows: more row blocks than a grid holds");
+  if (block > 0 && !one_rotation(M, K, block)) return decline("many rows: more to rotate than a launch holds");
   if (!workspace || workspace_bytes < ishz_affine_rows_workspace_size(M, K, N))
     return einval("workspace too small (ishz_affine_rows_workspace_size)");
   hipStream_t st = S(stream);

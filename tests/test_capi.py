@@ -32,6 +32,25 @@ def test_declines_without_touching_the_gpu():
     assert "declined" in _lib.last_error()
 
 
+def test_many_rows_decline_more_to_rotate_than_a_launch_holds():
+    """A rotation launches a workgroup of 256 threads per 512 values (Hadamard blocks above 128: per block) and a
+    launch holds less than 2^32 threads; one row fewer is asked for its workspace."""
+    L, p = _lib.lib(), ctypes.c_void_p(4096)
+
+    def affine(M, K, block):
+        return L.ishz_affine_linear_rows(p, _lib.DT_F16, M, K, p, block, p, p, p, _lib.DT_F16, 128, 4, 64, p, None, 0, None)
+
+    def exl3(M, K, N):
+        return L.ishz_exl3_apply_rows(p, _lib.DT_BF16, M, K, p, p, p, N, 4, 0, p, None, 0, None)
+    past = 1 << 24  # workgroups
+    for call in (lambda M: affine(M, 4096, 128), lambda M: affine(M, 4096, 512), lambda M: exl3(M, 4096, 128),
+                 lambda M: exl3(M, 256, 4096)):
+        assert call(past // 8) == _lib.DECLINED
+        assert call(past // 8 - 1) == _lib.EINVAL
+    assert affine(65535 * 64, 4096, 0) == _lib.EINVAL  # nothing to rotate
+    assert affine(past // 16, 4096, 256) == _lib.DECLINED and affine(past // 16 - 1, 4096, 256) == _lib.EINVAL
+
+
 def test_modulemap_names_the_header():
     here = os.path.dirname(_lib.HEADER)
     text = open(os.path.join(here, "module.modulemap")).read()
