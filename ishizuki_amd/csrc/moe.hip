@@ -20,7 +20,8 @@
 //    up to 16 tokens every gate/up workgroup routes and places in its own LDS, so the route +
 //    place launch is skipped; past 64, routing and placement are two launches.
 //  * More than four tokens an expert (Q4_K, Q6_K): the same problems on the sixteen-row kernel
-//    (wgemm.h). From eight (affine experts of even widths): the many-row kernel (qgemm.h).
+//    (wgemm.h). From eight and more (affine experts of even widths, moe_many_tokens): the many-row
+//    kernel (qgemm.h).
 //  * Combine: the weighted fp32 sum per token.
 // Only routed experts' blocks are ever read.
 #include <algorithm>
@@ -1116,18 +1117,43 @@ struct QMoeDown : VMoeDown {
     by_act(bf, [&]<bool BF>() { r.o[c] = bits16<BF>(BF ? v * r.f : v); });
   }
 };
-// From 8 tokens an expert on (on average); the images' sums go where the gathered GEMVs keep their h.
+// Whether the many-row kernel is ahead of the quads of vgemm.h, which decode with fewer instructions and spread few
+// columns over more workgroups: from 8 tokens an expert (on average), from 16 and 20 where the narrower projection
+// has under 96 and 64 blocks of 128 columns in all experts. Up to 12 tokens in all an expert is one pass of the quads
+// however the tokens fall, ahead but for the largest experts; those of 6 and 8 bits, whose decode is longer here, come
+// from 10. us there / here, fp16, E experts top k of H x I:
+//   4 top 2, 2048x768 (48 blocks), 4 bits     8 tokens an expert 26 / 38, 16: 36 / 40, 24: 43 / 41
+//   8 top 2, 1024x512 (64), 4 bits            8: 24 / 30, 12: 31 / 31, 16: 34 / 32
+//   32 top 4, 2048x768 (384), 4 bits          8: 60 / 55, 12: 87 / 56; 8 bits 8: 77 / 66
+//   64 top 8, 2048x768 (768), 4 bits          8: 99 / 73; 8 bits 8: 101 / 112, 10: 107 / 113, 12: 138 / 114
+//   8 top 8, 2048x768 (96), 4 bits            8: 30 / 41, 12: 34 / 42, 16: 44 / 42
+//   8 top 8, 4096x4096 (256), 4 bits          8: 83 / 97, 10: 100 / 98, 12: 101 / 97
+// Over 1602 shapes the call is 2 % (root mean square) behind the faster of the two; with one line at 8, 7 %.
+constexpr bool moe_many_tokens(int bits, int T, int k, int H, int E, int I) {
+  const size_t blocks = (size_t)E * std::min(2 * I, H) / 128;
+  const bool large = (size_t)E * H * I >= 100000000;
+  const int from = blocks < 64 ? 20 : blocks < 96 ? 16 : large && bits > 4 ? 10 : 8;
+  return (T > 12 || large) && (size_t)T * k >= (size_t)from * E;
+}
+static_assert(!moe_many_tokens(4, 39, 2, 2048, 4, 768) && moe_many_tokens(4, 40, 2, 2048, 4, 768) &&
+                  !moe_many_tokens(4, 63, 2, 1024, 8, 512) && moe_many_tokens(4, 64, 2, 1024, 8, 512) &&
+                  !moe_many_tokens(8, 79, 8, 2048, 64, 768) && moe_many_tokens(8, 80, 8, 2048, 64, 768) &&
+                  moe_many_tokens(4, 64, 8, 2048, 64, 768) && !moe_many_tokens(4, 12, 8, 2048, 8, 768) &&
+                  moe_many_tokens(4, 13, 8, 2048, 8, 768) && moe_many_tokens(4, 8, 8, 4096, 8, 4096),
+              "the lines above");
+// (the images' sums go where the gathered GEMVs keep their h)
 static bool moe_many_rows(int bits, int T, int H, int E, int I, int k, const AffPack &g, const AffPack &u, const AffPack &d,
                           const void *ws) {
   auto direct = [](const AffPack &p) { return lds_loadable(p.codes) && (uintptr_t)p.scales % 4 == 0 && (uintptr_t)p.biases % 4 == 0; };
-  return bits % 2 == 0 && direct(g) && direct(u) && direct(d) && lds_loadable(ws) && (size_t)T * k >= (size_t)8 * E && (size_t)T * (H / 256) * 16 <= (size_t)T * k * 2 * I * 2;
+  return bits % 2 == 0 && direct(g) && direct(u) && direct(d) && lds_loadable(ws) &&
+         moe_many_tokens(bits, T, k, H, E, I) && (size_t)T * (H / 256) * 16 <= (size_t)T * k * 2 * I * 2;
 }
 
 template <class F>
 struct QOf;
 template <int BITS, int GS, bool BF16S>
 struct QOf<FAffineN<BITS, GS, BF16S>> {
-  static constexpr bool EVEN = BITS % 2 == 0;
+  static constexpr int bits = BITS;
   using type = QAffine<BITS, GS, BF16S>;
 };
 
@@ -1157,8 +1183,8 @@ static int moe_ffn_affine(const void *x, int T, int H, int E, int I, int k, cons
     return launch_gemv<FMoeDownA<F>>(da, h16, y, st);
   }
   const int tiles_gu = 2 * ((I + 15) / 16), tiles_dn = (H + 15) / 16;
-  if constexpr (QOf<F>::EVEN)
-    if (moe_many_rows(2, T, H, E, I, k, gate, up, down, ma.ximg)) {  // x: as the caller gave it
+  if constexpr (QOf<F>::bits % 2 == 0)
+    if (moe_many_rows(QOf<F>::bits, T, H, E, I, k, gate, up, down, ma.ximg)) {  // x: as the caller gave it
       using Q = typename QOf<F>::type;
       const int dt = ma.bf ? ISHZ_DT_BF16 : ISHZ_DT_F16, P = T * k;
       const int mbs = std::min((T + 63) / 64, (4 * P / E + 63) / 64);  // row blocks for four times an even share

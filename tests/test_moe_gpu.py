@@ -413,13 +413,15 @@ def dense_reference(x, ids, w, gate, up, down):
     (4, 64, torch.float16, 70, 4, 2, 512, 256), (4, 128, torch.bfloat16, 130, 8, 4, 256, 512),
     (2, 64, torch.float16, 40, 4, 1, 256, 256), (8, 64, torch.bfloat16, 33, 4, 4, 512, 256),
     (6, 64, torch.float16, 300, 4, 2, 256, 256), (3, 64, torch.float16, 70, 4, 2, 256, 256),
-    (4, 64, torch.float16, 300, 32, 2, 256, 256), (4, 64, torch.bfloat16, 300, 32, 2, 512, 256),
-    (8, 128, torch.float16, 260, 64, 3, 256, 512)])
+    (2, 64, torch.float16, 100, 4, 1, 256, 256), (2, 128, torch.bfloat16, 60, 48, 8, 512, 512),
+    (8, 64, torch.float16, 110, 48, 4, 512, 256), (4, 64, torch.float16, 400, 32, 2, 256, 256),
+    (4, 64, torch.bfloat16, 300, 32, 2, 512, 256), (8, 128, torch.float16, 350, 64, 3, 256, 512)])
 @pytest.mark.parametrize("one_expert", [False, True])
 def test_swiglu_affine_many_tokens(bits, group, dt, T, E, k, H, I, one_expert):
-    """Eight tokens an expert and more: the many-row kernel (even widths), experts of one row tile and of
-    several row blocks, every token on the same experts, routing in launches of its own past 64 tokens. The last
-    three launch one or two row blocks and need five on those experts, so a workgroup takes several in turn."""
+    """Eight tokens an expert and more: the many-row kernel (even widths; from 8, 10, 16 or 20 by shape), experts of
+    one row tile and of several row blocks, every token on the same experts, routing in launches of its own past 64
+    tokens. The last three launch one or two row blocks and need five and more on those experts, so a workgroup
+    takes several in turn."""
     ex, (gate, up, down) = dense_affine_experts(E, H, I, bits, group, seed=bits + T)
     x = torch.from_numpy(np.random.default_rng(T).standard_normal((T, H)).astype(np.float32)).to(dt)
     logits = np.random.default_rng(T + 1).standard_normal((T, E)).astype(np.float32)
