@@ -37,10 +37,6 @@ def hadamard_rotate(x, block, signs=None, inverse=False):
     return y.reshape(shape)
 
 
-def _args(weight, scales, biases):
-    return (ptr(weight), ptr(scales), ptr(biases), DTYPES.get(scales.dtype, -1))
-
-
 def _check_width(N, K, x, weight, scales, biases, group_size, bits):
     """The C calls take K from x and step through the pack by it, so a pack of another width would be read
     past its end, or in the wrong rows. What they decline is left to them. (A pack that fits is told first: 0.6 us.)"""
@@ -63,9 +59,9 @@ def quantized_matmul(x, weight, scales, biases, group_size=64, bits=2):
     N = weight.shape[0]
     _check_width(N, K, x, weight, scales, biases, group_size, bits)
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    w, s, b, sdt = _args(weight, scales, biases)
-    rc = _lib.lib().ishz_affine_matmul(ptr(x), DTYPES.get(x.dtype, -1), M, K, w, s, b, sdt, N, bits,
-                                       group_size, ptr(y), stream())
+    rc = _lib.lib().ishz_affine_matmul(x.data_ptr(), DTYPES.get(x.dtype, -1), M, K, weight.data_ptr(), scales.data_ptr(),
+                                       biases.data_ptr(), DTYPES.get(scales.dtype, -1), N, bits, group_size, y.data_ptr(),
+                                       stream())
     return y if _lib.check(rc, "affine_matmul") else None
 
 
@@ -92,15 +88,18 @@ def linear(x, weight, scales, biases, signs=None, block=0, group_size=64, bits=2
     _check_width(N, K, x, weight, scales, biases, group_size, bits)
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     L = _lib.lib()
-    # (one fp16 row of a 2-bit pack is rotated and staged in the GEMV)
-    in_gemv = M == 1 and bits == 2 and group_size in (64, 128) and x.dtype is torch.float16
-    image = M > 1 and x.dtype is torch.bfloat16  # two and more bf16 rows: their fp16 image
-    ws_bytes = L.ishz_affine_workspace_size(M, K) if image or (block and _prestage and not in_gemv) else 0
+    if M > 1 and x.dtype is torch.bfloat16:  # their fp16 image
+        needs = True
+    elif block:  # (one fp16 row of a 2-bit pack is rotated and staged in the GEMV)
+        needs = _prestage and not (M == 1 and bits == 2 and group_size in (64, 128) and x.dtype is torch.float16)
+    else:
+        needs = False
+    ws_bytes = L.ishz_affine_workspace_size(M, K) if needs else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     s = device_f32(signs, x) if block else None
-    w, sc, b, sdt = _args(weight, scales, biases)
-    rc = L.ishz_affine_linear(ptr(x), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, w, sc, b, sdt, N,
-                              bits, group_size, ptr(y), ptr(ws), ws_bytes, stream())
+    rc = L.ishz_affine_linear(x.data_ptr(), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, weight.data_ptr(),
+                              scales.data_ptr(), biases.data_ptr(), DTYPES.get(scales.dtype, -1), N, bits, group_size,
+                              y.data_ptr(), ptr(ws), ws_bytes, stream())
     return y if _lib.check(rc, "affine_linear") else None
 
 
@@ -114,12 +113,13 @@ def linear_rows(x, weight, scales, biases, signs=None, block=0, group_size=64, b
     _check_width(N, K, x, weight, scales, biases, group_size, bits)
     L = _lib.lib()
     # what the library declines by these is declined before anything is allocated
-    takes = x.dtype in (torch.float16, torch.bfloat16) and K % 256 == 0 and bits in (2, 4, 6, 8) and group_size in (64, 128)
+    takes = (K % 256 == 0 and (x.dtype is torch.float16 or x.dtype is torch.bfloat16) and bits in (2, 4, 6, 8)
+             and (group_size == 64 or group_size == 128))
     ws_bytes = L.ishz_affine_rows_workspace_size(M, K, N) if takes else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if takes else None
     y = torch.empty((M, N), dtype=x.dtype, device=x.device) if takes else None
     s = device_f32(signs, x) if block else None
-    w, sc, b, sdt = _args(weight, scales, biases)
-    rc = L.ishz_affine_linear_rows(ptr(x), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, w, sc, b, sdt, N, bits,
-                                   group_size, ptr(y), ptr(ws), ws_bytes, stream())
+    rc = L.ishz_affine_linear_rows(x.data_ptr(), DTYPES.get(x.dtype, -1), M, K, ptr(s), block, weight.data_ptr(),
+                                   scales.data_ptr(), biases.data_ptr(), DTYPES.get(scales.dtype, -1), N, bits, group_size,
+                                   ptr(y), ptr(ws), ws_bytes, stream())
     return y if _lib.check(rc, "affine_linear_rows") else None

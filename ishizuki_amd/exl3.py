@@ -54,19 +54,19 @@ def rotate(x, scales, before, out_dtype):
     return y
 
 
-def _check_width(x, t):
-    """The C calls take K from the tensor, so a narrower x would be read past its end."""
-    if x.dim() != 2 or x.shape[1] != t.input_dim:
-        raise _lib.IshzError(f"x of shape {tuple(x.shape)} through an EXL3 tensor of width {t.input_dim}")
+def _rows(shape, t):
+    """Rows of x. The C calls take K from the tensor, so a narrower x would be read past its end."""
+    if len(shape) != 2 or shape[1] != t.input_dim:
+        raise _lib.IshzError(f"x of shape {tuple(shape)} through an EXL3 tensor of width {t.input_dim}")
+    return shape[0]
 
 
 def matvec(xh, t, workspace=None):
     """xh [M, K] (already rotated; fp16, bf16 or fp32) -> fp32 [M, N]. With `workspace` (a uint8
     device tensor of matvec_workspace_size bytes) the call allocates nothing."""
     require_cuda(xh, t.trellis)
-    _check_width(xh, t)
+    M = _rows(xh.shape, t)
     xh = xh.contiguous()
-    M = xh.shape[0]
     y = torch.empty((M, t.output_dim), dtype=torch.float32, device=xh.device)
     L = _lib.lib()
     if workspace is None:
@@ -103,15 +103,15 @@ def apply_rows(x, t):
     """EXL3Kernels.apply for a prompt: any number of rows [M, K] in one call; None if declined (fp32 x,
     K not a multiple of 256), where `apply` takes 16 rows at a time."""
     require_cuda(x, t.trellis)
-    _check_width(x, t)
+    M = _rows(x.shape, t)
     x = x.contiguous()
-    M = x.shape[0]
     L = _lib.lib()
     # what the library declines by these is declined before anything is allocated
-    takes = x.dtype in (torch.float16, torch.bfloat16) and t.input_dim % 256 == 0
-    ws_bytes = L.ishz_exl3_rows_workspace_size(M, t.input_dim, t.output_dim) if takes else 0
+    K, N = t.input_dim, t.output_dim
+    takes = K % 256 == 0 and (x.dtype is torch.float16 or x.dtype is torch.bfloat16)
+    ws_bytes = L.ishz_exl3_rows_workspace_size(M, K, N) if takes else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if takes else None
-    y = torch.empty((M, t.output_dim), dtype=x.dtype, device=x.device) if takes else None
-    rc = L.ishz_exl3_apply_rows(ptr(x), DTYPES.get(x.dtype, -1), M, t.input_dim, ptr(t.trellis), ptr(t.suh), ptr(t.svh),
-                                t.output_dim, t.bits2, t.codebook, ptr(y), ptr(ws), ws_bytes, stream())
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device) if takes else None
+    rc = L.ishz_exl3_apply_rows(x.data_ptr(), DTYPES.get(x.dtype, -1), M, K, t.trellis.data_ptr(), t.suh.data_ptr(),
+                                t.svh.data_ptr(), N, t.bits2, t.codebook, ptr(y), ptr(ws), ws_bytes, stream())
     return y if _lib.check(rc, "exl3_apply_rows") else None
