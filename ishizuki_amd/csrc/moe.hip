@@ -997,7 +997,7 @@ static int moe_route_all(const float *logits, int T, int E, int topk, int normal
   const int nr = std::min((T + 3) / 4 * 4, 64);  // routing rows: whole waves, at most 16
   const size_t fused_lds = ((size_t)nr * route_row_words(E, topk) + E + (size_t)T * topk) * 4;
   if (!place) return route_launch(logits, T, E, topk, normalize, R, st);
-  // (one workgroup routes 64 tokens at a time, about 4 us a round; 512 tokens took 56 us)
+  // (one workgroup routes 64 tokens at a time, about 7 us a round: 512 tokens took 56 us)
   if (T <= 64 && fused_lds <= 64 * 1024) {
     hipLaunchKernelGGL(moe_route_place_kernel, dim3(1), dim3(16 * nr), fused_lds, st, logits, T, E, topk, normalize, R);
     ISHZ_LAUNCH_CHECK("moe route launch");

@@ -75,7 +75,8 @@ class PackedLinear:
         One call is ahead of 16-row calls from 17 rows on (us in a replayed graph, 16-row calls / one call, 17
         rows: 17408x5120 2-bit rotated 55.7 / 34.3, 4-bit 56.2 / 34.8, 8-bit 64.9 / 46.2, EXL3 2-bit 58.2 / 41.5;
         1024x4096 21.5 / 19.5, 20.3 / 18.4, 22.2 / 20.9, 29.9 / 22.3), but for weights of about a million: 1024x1024
-        4-bit 15.0 / 15.7, 8-bit 15.1 / 17.8. Called from Python those take 26 / 16, so there is no other line."""
+        4-bit 15.0 / 15.7, 8-bit 15.1 / 17.8, EXL3 6-bit 29 / 36. Called from Python those take 26 / 16 and 49 / 36, so
+        there is no other line."""
         n = rows.shape[0]
         if n <= 16:
             return None
